@@ -43,6 +43,19 @@ struct LdsStack {
 // SEG: holds a leaf segment to evaluate; DONE: the queue is drained.
 enum SlotState : uint32_t { SLOT_EMPTY = 0, SLOT_RAY = 1, SLOT_SEG = 2, SLOT_DONE = 3, SLOT_NEW = 4 };
 
+// N-BVH nodes copied into LDS per workgroup (the first ones: the top of the breadth-first tree,
+// all of it for up to this many nodes); 16 KB for 512 nodes keeps two workgroups per CU.
+constexpr uint32_t kNodeCache = 512;
+
+// Copy the first min(n_nodes, kNodeCache) nodes into LDS (the caller synchronises).
+__device__ __forceinline__ uint32_t stage_nodes(const NetArgs& a, uint4* lds)
+{
+    const uint32_t n = a.n_nodes < kNodeCache ? a.n_nodes : kNodeCache;
+    const uint4* src = reinterpret_cast<const uint4*>(a.nodes);
+    for (uint32_t i = threadIdx.x; i < 2 * n; i += blockDim.x) lds[i] = src[i];
+    return n;
+}
+
 // Per-ray result of a neural query, built up segment by segment (shared by the persistent wave
 // scheduler and the sorted wavefront rounds, so both make identical decisions).
 struct HitState {
@@ -223,6 +236,17 @@ struct RayQueue {
         return (block * 8u + (w >> 3)) * image_width + tile * 8u + (w & 7u);
     }
 };
+
+// Slots a wave of a persistent launch fills: all 64 once the rays would fill them, else the rays
+// spread evenly over the launch's waves (at least kMinWaveSlots each), so that a small batch uses
+// every CU's L1 and miss queue instead of a few. The count may live on the device, so the kernel
+// decides; the host sizes the grid (query_blocks, kernels/launch.h).
+__device__ __forceinline__ uint32_t wave_slots(uint32_t n_rays)
+{
+    const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+    const uint32_t even  = n_rays / waves + (n_rays % waves != 0u ? 1u : 0u);
+    return even < kMinWaveSlots ? kMinWaveSlots : (even < 64u ? even : 64u);
+}
 
 // Phase A. Returns false when the wave has no segment left to evaluate (all slots DONE).
 // Traversal rounds: every slot still looking for a leaf advances at most kTraversalBudget nodes

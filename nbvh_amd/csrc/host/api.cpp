@@ -74,34 +74,6 @@ void DevBuf::alloc(nbvh_ctx* c, size_t n)
     ctx->used += n;
 }
 
-namespace {
-
-// MLP layout consumed by the FP32 kernels: layers 1, 3, 5 row-major, layers 2, 4 transposed.
-std::vector<float> fp32_kernel_layout(const nbvh_network_config& cfg, const std::vector<float>& mlp)
-{
-    const uint32_t K0 = cfg.n_points * cfg.grid.n_levels * cfg.grid.n_features_per_level;
-    std::vector<float> out(mlp.size());
-    size_t off = 0;
-    uint32_t in = K0;
-    for (uint32_t layer = 0; layer <= cfg.n_hidden_layers; layer++) {
-        const uint32_t o = layer == cfg.n_hidden_layers ? cfg.n_outputs : cfg.n_neurons;
-        const bool transposed = (layer % 2 == 1) && layer != cfg.n_hidden_layers;
-        for (uint32_t j = 0; j < o; j++)
-            for (uint32_t k = 0; k < in; k++) {
-                const float w = mlp[off + (size_t)j * in + k];
-                if (transposed)
-                    out[off + (size_t)k * o + j] = w;
-                else
-                    out[off + (size_t)j * in + k] = w;
-            }
-        off += (size_t)o * in;
-        in = cfg.n_neurons;
-    }
-    return out;
-}
-
-}  // namespace
-
 void refresh_args(nbvh_scene* s)
 {
     NetArgs& a = s->args;
@@ -180,7 +152,7 @@ void upload_network(nbvh_scene* s)
     std::vector<uint16_t> t16(s->tables.size());
     for (size_t i = 0; i < t16.size(); i++) t16[i] = float_to_half(s->tables[i] * s->table_scale);
     s->d_tables16.upload(ctx, t16.data(), t16.size());
-    const auto k32 = fp32_kernel_layout(s->cfg, s->mlp);
+    const auto k32 = f32_fragments(s->cfg, s->mlp);
     s->d_mlp32.upload(ctx, k32.data(), k32.size());
     MfmaWeights mw = mfma_weight_layout(s->cfg, s->mlp);
     s->d_frag.upload(ctx, mw.frag16.data(), mw.frag16.size());
@@ -390,7 +362,7 @@ void run_query_wavefront(nbvh_ctx* ctx, const nbvh_scene* s, const nbvh_query_pa
             hip_check(wf_encode(a, batch, segs, U32(o_order), m, in, stream), "wavefront encode");
             bool supported = false;
             if (p->precision == NBVH_PREC_FP32)
-                hip_check(network_fp32(a, in, m, nullptr, logits, stream, &supported), "fp32 network");
+                hip_check(network_fp32(a, in, m, nullptr, logits, (uint32_t)ctx->n_cus, stream, &supported), "fp32 network");
             else
                 hip_check(network_mfma(a, p->precision, in, m, nullptr, logits, (uint32_t)ctx->n_cus, stream, &supported), "mfma network");
             if (!supported) fail(NBVH_ERR_UNSUPPORTED, "no network kernel for this network shape / precision");
@@ -463,7 +435,8 @@ void run_network(nbvh_ctx* ctx, const nbvh_scene* s, uint32_t precision, const f
     hip_check(hipSetDevice(ctx->device), "hipSetDevice");
     bool supported = false;
     if (precision == NBVH_PREC_FP32)
-        hip_check(network_fp32(s->args, d_in, n, d_out, d_logits, stream, &supported), "fp32 network");
+        hip_check(network_fp32(s->args, d_in, n, d_out, d_logits, (uint32_t)ctx->n_cus, stream, &supported),
+                  "fp32 network");
     else
         hip_check(network_mfma(s->args, precision, d_in, n, d_out, d_logits, (uint32_t)ctx->n_cus, stream,
                                &supported), "mfma network");

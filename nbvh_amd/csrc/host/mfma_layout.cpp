@@ -82,4 +82,33 @@ MfmaWeights mfma_weight_layout(const nbvh_network_config& cfg, const std::vector
     return out;
 }
 
+std::vector<float> f32_fragments(const nbvh_network_config& cfg, const std::vector<float>& mlp)
+{
+    const uint32_t K0 = cfg.n_points * cfg.grid.n_levels * cfg.grid.n_features_per_level;
+    std::vector<float> out;
+    if (cfg.n_neurons != 64 || cfg.n_hidden_layers != 4 || cfg.n_outputs != 8 || K0 % 4 != 0) return out;
+    out.resize(mlp.size());
+    size_t off = 0;
+    uint32_t in = K0;
+    for (uint32_t layer = 0; layer < 4; layer++) {
+        const uint32_t steps = in / 2;
+        for (uint32_t rb = 0; rb < 2; rb++)
+            for (uint32_t s = 0; s < steps; s++)
+                for (uint32_t lane = 0; lane < 64; lane++) {
+                    // Row l % 32 = 8 q + 4 g + i of the block holds neuron 2 (16 rb + 4 q + i) + g.
+                    const uint32_t row = lane % 32, q = row / 8, g = (row / 4) % 2, i = row % 4;
+                    const uint32_t n = 2 * (16 * rb + 4 * q + i) + g, k = 2 * s + lane / 32;
+                    out[off + ((size_t)(rb * (steps / 2) + s / 2) * 64 + lane) * 2 + s % 2] =
+                        mlp[off + (size_t)n * in + k];
+                }
+        off += (size_t)64 * in;
+        in = 64;
+    }
+    for (uint32_t s = 0; s < 32; s++)
+        for (uint32_t g = 0; g < 2; g++)
+            for (uint32_t row = 0; row < 8; row++)
+                out[off + ((size_t)(s / 2 * 2 + g) * 8 + row) * 2 + s % 2] = mlp[off + (size_t)row * 64 + 2 * s + g];
+    return out;
+}
+
 }  // namespace nbvh

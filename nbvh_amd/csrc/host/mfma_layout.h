@@ -28,6 +28,10 @@ inline uint32_t mfma_h_k(uint32_t g, uint32_t s, uint32_t e)
     return 32 * (s / 2) + 16 * (s % 2) + 8 * (e / 4) + 4 * g + (e % 4);
 }
 
+// Weights as v_mfma_f32_32x32x2_f32 A operands (device/mlp_f32.h), or nothing where no kernel
+// evaluates the shape (H != 64, other than 4 hidden layers, inputs not in pairs of k-steps).
+std::vector<float> f32_fragments(const nbvh_network_config& cfg, const std::vector<float>& mlp);
+
 MfmaWeights mfma_weight_layout(const nbvh_network_config& cfg, const std::vector<float>& mlp);
 
 }  // namespace nbvh

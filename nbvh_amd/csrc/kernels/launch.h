@@ -7,6 +7,35 @@
 
 namespace nbvh {
 
+// Resident workgroups per CU of a kernel (1 if the runtime does not say).
+template <typename K>
+inline uint32_t blocks_per_cu(K kernel, uint32_t threads)
+{
+    int b = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, reinterpret_cast<const void*>(kernel), (int)threads, 0) !=
+            hipSuccess ||
+        b <= 0) {
+        (void)hipGetLastError();
+        b = 1;
+    }
+    return (uint32_t)b;
+}
+
+// Workgroups of a persistent query over n rays, at most max_blocks: a batch too small to fill
+// their slots is spread over as many as get kMinWaveSlots rays per wave (wave_slots,
+// device/wave_query.h).
+inline uint32_t query_blocks(uint32_t n, uint32_t waves_per_block, uint32_t max_blocks)
+{
+    const uint32_t per_block = waves_per_block * kMinWaveSlots;
+    const uint32_t blocks    = n / per_block + (n % per_block != 0u ? 1u : 0u);
+    return blocks < max_blocks ? blocks : max_blocks;
+}
+
+// Dense-prefix length the kernels are specialised for (the hash-only gather of levels >= it):
+// 4 covers the 1024x1024 workload's grid (16 levels, base 16, scale 1.5, 2^19) and the chess
+// configuration (8 levels, base 8, scale 2, 2^18). Other grids take the general gather (ND = -1).
+constexpr int kDensePrefix = 4;
+
 // Primary rays (camera_raygen with LCG jitter).
 hipError_t raygen(const nbvh_camera& cam, uint32_t w, uint32_t h, uint32_t sample, uint32_t frame, nbvh_ray* rays,
                   hipStream_t stream);
@@ -82,8 +111,8 @@ hipError_t query_triangles(const TriArgs& a, const RayBatch& rb, hipStream_t str
 // *supported = false when no kernel instance matches the network shape.
 hipError_t query_fp32(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus, hipStream_t stream,
                       bool* supported);
-hipError_t network_fp32(const NetArgs& a, const float* in, uint32_t n, float* out, float* logits, hipStream_t stream,
-                        bool* supported);
+hipError_t network_fp32(const NetArgs& a, const float* in, uint32_t n, float* out, float* logits, uint32_t n_cus,
+                        hipStream_t stream, bool* supported);
 
 // MFMA paths: precision = NBVH_PREC_FP16 / BF16 / FP8.
 hipError_t query_mfma(const NetArgs& a, uint32_t precision, const RayBatch& rb, uint32_t* queue, uint32_t n_cus,

@@ -11,6 +11,7 @@
 //     v_permlane32_swap per register pair moves the halves into the operand layout.
 #include <hip/hip_runtime.h>
 
+#include "../device/grid_gather.h"
 #include "../device/wave_query.h"
 #include "launch.h"
 
@@ -105,31 +106,17 @@ __device__ __forceinline__ void load_corner(__amdgpu_buffer_rsrc_t tab, uint32_t
 // hardware range check returns 0 for any offset past the table instead of faulting. Levels are
 // processed in groups of G: all corner offsets of the group, then all its loads, then the
 // corner weights and the FP32 accumulation over corners 0..7 (tcnn's trilinear weights).
-// Byte offsets of the 8 corners of one level at point (x, y, z), and the fractional position.
-// HASHED: the level is hashed (a power-of-two size), so only the coherent prime hash is formed:
-// two multiplies per level, then one xor-and and one add-shift per corner. The hash of any
-// position is in range, so this form is exact for points outside the unit cube too. Otherwise
-// the general form (dense or hashed at run time, grid_corners) with its EXACT modulo switch.
+// Byte offsets of the 8 corners of one level at point (x, y, z) in the whole FP16 table, and the
+// fractional position (level_entries: HASHED and EXACT).
 template <int F, bool HASHED, bool EXACT>
 __device__ __forceinline__ void level_offsets(const GridLevel& lv, float x, float y, float z, uint32_t off[8],
                                               float fr[3])
 {
-    uint32_t g[3];
-    grid_cell(lv, x, y, z, g, fr);
     constexpr uint32_t kShift = F == 2 ? 2u : 3u;  // log2 of the entry bytes (F halves)
-    if constexpr (HASHED) {
-        const uint32_t hy0 = g[1] * 2654435761u, hy1 = hy0 + 2654435761u;
-        const uint32_t hz0 = g[2] * 805459861u, hz1 = hz0 + 805459861u;
-        const uint32_t yz[4] = {hy0 ^ hz0, hy1 ^ hz0, hy0 ^ hz1, hy1 ^ hz1};
-        const uint32_t mask = lv.size - 1u, x1 = g[0] + 1u;
+    uint32_t idx[8];
+    level_entries<HASHED, EXACT>(lv, x, y, z, idx, fr);
 #pragma unroll
-        for (int c = 0; c < 8; c++) off[c] = (((((c & 1) ? x1 : g[0]) ^ yz[c >> 1]) & mask) + lv.offset) << kShift;
-    } else {
-        uint32_t idx[8];
-        grid_corners<EXACT>(lv, g, idx);
-#pragma unroll
-        for (int c = 0; c < 8; c++) off[c] = (idx[c] + lv.offset) << kShift;
-    }
+    for (int c = 0; c < 8; c++) off[c] = (idx[c] + lv.offset) << kShift;
 }
 
 // One group of G levels of point p: all 8G corner offsets, then all 8G loads, then the corner
@@ -167,7 +154,7 @@ __device__ __forceinline__ void gather_group(const NetArgs& a, __amdgpu_buffer_r
         for (int k = 0; k < F; k++) acc[k] = 0.f;
 #pragma unroll
         for (int c = 0; c < 8; c++) {
-            const float w = (wx[c & 1] * wy[(c >> 1) & 1]) * wz[c >> 2];
+            const float w = trilinear_weight(c, wx, wy, wz);
 #pragma unroll
             for (int k = 0; k < F; k++) {
                 const uint32_t bits = (k & 1) ? (q[i][c][k / 2] >> 16) : (q[i][c][k / 2] & 0xFFFFu);
@@ -494,22 +481,6 @@ __device__ __forceinline__ void mfma_network_fp8(const NetArgs& a, const Fp8Lds<
     gather_logits(out, g, 1.f / cum[g], z);
 }
 
-// N-BVH nodes copied into LDS per workgroup (the first ones: the top of the breadth-first tree,
-// all of it for up to this many nodes); 16 KB for 512 nodes keeps two workgroups per CU.
-#ifndef NBVH_NODE_CACHE
-#define NBVH_NODE_CACHE 512
-#endif
-constexpr uint32_t kNodeCache = NBVH_NODE_CACHE;
-
-// Copy the first min(n_nodes, kNodeCache) nodes into LDS (the caller synchronises).
-__device__ __forceinline__ uint32_t stage_nodes(const NetArgs& a, uint4* lds)
-{
-    const uint32_t n = a.n_nodes < kNodeCache ? a.n_nodes : kNodeCache;
-    const uint4* src = reinterpret_cast<const uint4*>(a.nodes);
-    for (uint32_t i = threadIdx.x; i < 2 * n; i += blockDim.x) lds[i] = src[i];
-    return n;
-}
-
 // Waves per workgroup of the query kernel; the workgroup shares one LDS copy of the weights.
 #ifndef NBVH_MFMA_BLOCK_WAVES
 #define NBVH_MFMA_BLOCK_WAVES 4
@@ -528,7 +499,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void n
     constexpr int NF = MlpShape<P * L * F>::N_FRAG;
     __shared__ uint4 wfrag[NF * 64];
     __shared__ uint32_t stack_lds[kWavesPerBlock * kNeuralStackSize * 64];
-    __shared__ uint4 node_lds[2 * (kNodeCache > 0 ? kNodeCache : 1)];
+    __shared__ uint4 node_lds[2 * kNodeCache];
     const uint32_t n_cached = stage_nodes(a, node_lds);
     stage_weights<P, L, F, BF16>(a, wfrag);  // ends with the barrier
     const CachedNodes nodes{a.nodes, node_lds, n_cached};
@@ -586,7 +557,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void n
 {
     __shared__ Fp8Lds<P * L * F> w;
     __shared__ uint32_t stack_lds[kWavesPerBlock * kNeuralStackSize * 64];
-    __shared__ uint4 node_lds[2 * (kNodeCache > 0 ? kNodeCache : 1)];
+    __shared__ uint4 node_lds[2 * kNodeCache];
     const uint32_t n_cached = stage_nodes(a, node_lds);
     stage_weights_fp8<P * L * F>(a, w);  // ends with the barrier
     const CachedNodes nodes{a.nodes, node_lds, n_cached};
@@ -637,22 +608,6 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void network_fp8_kernel(NetArg
 }  // namespace dev
 
 namespace {
-
-template <typename K>
-uint32_t blocks_per_cu(K kernel, uint32_t threads)
-{
-    int b = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, kernel, (int)threads, 0) != hipSuccess || b <= 0) {
-        (void)hipGetLastError();
-        b = 1;
-    }
-    return (uint32_t)b;
-}
-
-// Dense-prefix length the kernels are specialised for (the hash-only gather of levels >= it):
-// 4 covers the 1024x1024 workload's grid (16 levels, base 16, scale 1.5, 2^19) and the chess
-// configuration (8 levels, base 8, scale 2, 2^18). Other grids take the general gather (ND = -1).
-constexpr int kDensePrefix = 4;
 
 template <int P, int L, int F, bool BF16, bool PARTS, int ND>
 hipError_t launch_query_k(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus, hipStream_t stream)

@@ -16,6 +16,7 @@ constexpr float    kInferenceMaxtEps   = 1e-3f;  // neural_bvh_renderer_constant
 constexpr float    kDepthEpsilon       = 0.2f;   // neural_bvh_module.h:270
 constexpr float    kFixedDepthEpsilon  = 1e-5f;  // neural_bvh_module.h:271
 constexpr uint32_t kDefaultMaxSteps    = 1000;   // m_max_traversal_steps, neural_bvh_module.h:200
+constexpr uint32_t kMinWaveSlots       = 4;      // fewest rays per wave a small query is spread over
 
 // One level of the multiresolution grid (tcnn GridEncoding, public convention).
 struct GridLevel {
@@ -49,7 +50,7 @@ struct NetArgs {
     uint32_t tables_f16_bytes;         // size of tables_f16 (< 2^31: buffer-resource range)
     float    table_scale;              // power of two
     float    inv_table_scale;
-    const float*    mlp_f32;           // row-major matrices, concatenated
+    const float*    mlp_f32;           // FP32 MFMA fragments (f32_fragments, host/mfma_layout.cpp)
     const uint16_t* mlp_frag;          // MFMA fragment-ordered half/bf16 weights
     const uint8_t*  mlp_frag_fp8;      // FP8 e4m3 hidden-layer fragments
     float    fp8_wscale[8];            // per-layer weight dequantisation scales (FP8 variant)

@@ -113,6 +113,43 @@ def test_network_fp32_bit_exact(nb, orc, bench):
     assert np.array_equal(out, o32.astype(np.float32))
 
 
+@pytest.mark.parametrize("levels,features", [(16, 2), (8, 4), (4, 2), (2, 2)])
+def test_network_fp32_bit_exact_at_tile_edges(nb, orc, ctx, bench, levels, features):
+    """Every input width of the FP32 matrix-core network (96, 96, 24, 12) at the edges of a wave
+    (64) and a workgroup (512), with weights that reach the subnormal range and exact zeros."""
+    scene = nb.Scene(ctx, bench["v"], bench["t"])
+    cfg = nb.network_config(n_levels=levels, n_features_per_level=features, log2_hashmap_size=14)
+    scene.init_network(cfg, seed=4, table_range=1e-2)
+    _, tables, mlp = scene.network()
+    tables[::7] = 0.0
+    tables[::11] *= np.float32(1e-37)
+    mlp[::13] = 0.0
+    mlp[::17] *= np.float32(1e-38)
+    scene.load_network_model(cfg, tables, mlp)
+    net = orc.Net(cfg, tables, mlp, *scene.bbox())
+    mod = nb.NeuralBVHModule(ctx, scene)
+    rng = np.random.default_rng(8)
+    x = rng.uniform(-0.05, 1.05, (1030, 9)).astype(np.float32)
+    _, z32 = net.network(x, mode=orc.FP32)
+    for n in (1, 31, 32, 33, 63, 64, 65, 511, 512, 513, 1030):
+        _, logits = mod.network_inference(x[:n], precision=nb.PREC_FP32)
+        assert np.array_equal(logits.view(np.uint32), z32[:n].astype(np.float32).view(np.uint32)), n
+    scene.close()
+
+
+@pytest.mark.parametrize("n", [1, 4, 5, 63, 65, 4097, 8193])
+@pytest.mark.parametrize("precision", ["fp32", "fp16", "bf16", "fp8"])
+def test_small_batches_equal_the_whole(nb, orc, bench, n, precision):
+    """A batch too small to fill the launch is spread over more waves with fewer rays each: the
+    records are those of the same rays inside a batch that fills it."""
+    prec = {"fp32": nb.PREC_FP32, "fp16": nb.PREC_FP16, "bf16": nb.PREC_BF16, "fp8": nb.PREC_FP8}[precision]
+    _, rays = camera_rays(nb, orc, 512, 400)
+    whole = bench["module"].neural_bvh_traversal(rays, precision=prec)
+    for start in (0, 100000):
+        part = bench["module"].neural_bvh_traversal(rays[start:start + n], precision=prec)
+        assert hits_equal(part, whole[start:start + n])
+
+
 @pytest.mark.parametrize("any_hit", [False, True])
 def test_neural_query_fp32_bit_exact(nb, orc, bench, any_hit):
     _, rays = camera_rays(nb, orc, 128, 128)
