@@ -35,5 +35,43 @@ __device__ __forceinline__ float trilinear_weight(int c, const float wx[2], cons
     return (wx[c & 1] * wy[(c >> 1) & 1]) * wz[c >> 2];
 }
 
+// How a wave gathers the features of its slots.
+//   LEVELS  every lane its own segment, level after level (the three points of a level together);
+//   PHASES  the same, the hashed levels in the order of level_phases;
+//   WIDE    few slots per wave: a lane takes one level of one slot, 64 / L slots at a time, so that
+//           a segment costs one memory round trip instead of one per level.
+enum class Gather { LEVELS, PHASES, WIDE };
+
+// Visit each of N levels once, f(level) with a wave-uniform level, starting with the level whose
+// turn it is: the turn moves every kLevelTicks of the 100 MHz clock, alike on every CU. The tables
+// of all hashed levels (2 MB each at 2^19 entries in FP16, 12 of them) are six times an XCD's 4 MB
+// L2, but one or two levels fit: waves that agree on the level share its lines there, and a wave
+// that falls behind skips ahead to the common level and returns to the others later.
+// Measured (us, gather order: all levels of a point / levels / phases): 1024 x 1024 camera rays
+// 1300 / 1258 / 1164, 4M incoherent rays 13143 / 12311 / 11310, FP32 camera rays 1760 / - / 1690,
+// 1M scattered segments in the network kernel, whose waves keep step by themselves, 2204 / 1685 /
+// 1800 and more. Ticks of 128 / 192 / 256 / 384 / 512: 1231 / 1179 / 1164 / 1170 / 1170 us.
+constexpr uint32_t kLevelTicks = 256;
+template <int N, typename Fn>
+__device__ __forceinline__ void level_phases(const Fn& f)
+{
+    static_assert(N >= 1 && N < 32, "one bit per level");
+    uint32_t left = (1u << N) - 1u;
+#pragma clang loop unroll(disable)
+    while (left != 0u) {
+        const uint32_t turn = ((uint32_t)__builtin_amdgcn_s_memrealtime() / kLevelTicks) % (uint32_t)N;
+        const uint32_t now  = (uint32_t)__builtin_amdgcn_readfirstlane((int)turn);
+        const uint32_t up   = left >> now;
+        const uint32_t l    = up != 0u ? now + (uint32_t)__builtin_ctz(up) : (uint32_t)__builtin_ctz(left);
+        left &= ~(1u << l);
+        f(l);
+    }
+}
+
+// Grids of fewer hashed levels gain nothing from phases (8 levels, 4 of them hashed: 402 us either
+// way on a 1013 x 691 frame), and their wider entries leave no registers for them.
+template <int L, int ND>
+constexpr Gather kQueryGather = ND >= 0 && L - ND >= 8 ? Gather::PHASES : Gather::LEVELS;
+
 }  // namespace dev
 }  // namespace nbvh

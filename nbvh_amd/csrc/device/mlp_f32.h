@@ -48,74 +48,128 @@ __device__ __forceinline__ void stage_weights_f32(const float* __restrict__ frag
     for (uint32_t i = threadIdx.x; i < (uint32_t)F32Layout<K0>::FLOATS / 4u; i += blockDim.x) lds[i] = src[i];
 }
 
-// Features of G levels of one point: all corner entries, then all loads, then the weights and the
-// accumulation over corners 0..7.
-template <int F, int G, bool HASHED, bool EXACT>
-__device__ __forceinline__ void gather_levels_f32(const NetArgs& a, const float* __restrict__ tables, const float* pt,
-                                                  int l0, float* x)
+// Features of one level for all P points: all corner entries, then all loads, then the weights and
+// the accumulation over corners 0..7. out[p * F + f].
+template <int P, int F, bool HASHED, bool EXACT>
+__device__ __forceinline__ void gather_level_f32(const GridLevel& lv, const float* __restrict__ tables,
+                                                 const float* pts, float* out)
 {
     typedef float entry_t __attribute__((ext_vector_type(F)));
-    uint32_t idx[G][8];
-    float fr[G][3];
+    uint32_t idx[P][8];
+    float fr[P][3];
 #pragma unroll
-    for (int i = 0; i < G; i++) level_entries<HASHED, EXACT>(a.level[l0 + i], pt[0], pt[1], pt[2], idx[i], fr[i]);
-    entry_t q[G][8];
+    for (int p = 0; p < P; p++)
+        level_entries<HASHED, EXACT>(lv, pts[3 * p], pts[3 * p + 1], pts[3 * p + 2], idx[p], fr[p]);
+    // A uniform base per level and a 32-bit byte offset in it (2^26 entries of 16 bytes at most).
+    const char* base = reinterpret_cast<const char*>(tables + (size_t)lv.offset * F);
+    entry_t q[P][8];
 #pragma unroll
-    for (int i = 0; i < G; i++) {
-        // A uniform base per level and a 32-bit byte offset in it (2^26 entries of 16 bytes at most).
-        const char* base = reinterpret_cast<const char*>(tables + (size_t)a.level[l0 + i].offset * F);
+    for (int p = 0; p < P; p++)
 #pragma unroll
         for (int c = 0; c < 8; c++)
-            q[i][c] = *reinterpret_cast<const entry_t*>(base + idx[i][c] * (uint32_t)sizeof(entry_t));
-    }
+            q[p][c] = *reinterpret_cast<const entry_t*>(base + idx[p][c] * (uint32_t)sizeof(entry_t));
 #pragma unroll
-    for (int i = 0; i < G; i++) {
-        const float wx[2] = {1.f - fr[i][0], fr[i][0]}, wy[2] = {1.f - fr[i][1], fr[i][1]};
-        const float wz[2] = {1.f - fr[i][2], fr[i][2]};
-        float acc[F];
+    for (int p = 0; p < P; p++) {
+        const float wx[2] = {1.f - fr[p][0], fr[p][0]}, wy[2] = {1.f - fr[p][1], fr[p][1]};
+        const float wz[2] = {1.f - fr[p][2], fr[p][2]};
 #pragma unroll
-        for (int k = 0; k < F; k++) acc[k] = 0.f;
+        for (int k = 0; k < F; k++) out[p * F + k] = 0.f;
 #pragma unroll
         for (int c = 0; c < 8; c++) {
             const float w = trilinear_weight(c, wx, wy, wz);
 #pragma unroll
-            for (int k = 0; k < F; k++) acc[k] = fmaf(w, q[i][c][k], acc[k]);
+            for (int k = 0; k < F; k++) out[p * F + k] = fmaf(w, q[p][c][k], out[p * F + k]);
         }
-#pragma unroll
-        for (int k = 0; k < F; k++) x[(l0 + i) * F + k] = acc[k];
     }
 }
 
-// Levels whose loads are issued together: 1, 2 and 4 measure alike (1791 / 1760 / 1757 us for the
-// 1024 x 1024 frame); 2 leaves the register allocator room.
-constexpr int kF32GatherGroup = 2;
-
-// ND >= 0: levels [ND, L) are hashed (n_dense == ND, checked at launch); ND < 0: any grid.
-template <int P, int L, int F, int ND, bool EXACT>
+// All features, x[p * L * F + l * F + f]. ND >= 0: levels [ND, L) are hashed (n_dense == ND,
+// checked at launch); ND < 0: any grid. G: the order of the levels.
+template <int P, int L, int F, int ND, bool EXACT, Gather G>
 __device__ __forceinline__ void gather_features_f32(const NetArgs& a, const float* __restrict__ tables,
                                                     const float* pts, float* x)
 {
-    constexpr int G = L % kF32GatherGroup == 0 ? kF32GatherGroup : 1;
 #pragma unroll
-    for (int p = 0; p < P; p++)
+    for (int l = 0; l < (ND >= 0 ? ND : L); l++) {
+        float r[P * F];
+        gather_level_f32<P, F, false, EXACT>(a.level[l], tables, pts, r);
 #pragma unroll
-        for (int l0 = 0; l0 < L; l0 += G) {
-            if (ND >= 0 && l0 >= ND)  // folded at compile time after unrolling
-                gather_levels_f32<F, G, true, false>(a, tables, pts + 3 * p, l0, x + p * L * F);
-            else
-                gather_levels_f32<F, G, false, EXACT>(a, tables, pts + 3 * p, l0, x + p * L * F);
+        for (int p = 0; p < P; p++)
+#pragma unroll
+            for (int k = 0; k < F; k++) x[(p * L + l) * F + k] = r[p * F + k];
+    }
+    if constexpr (ND >= 0 && G == Gather::PHASES) {
+        level_phases<L - ND>([&](uint32_t l) {
+            float r[P * F];
+            gather_level_f32<P, F, true, false>(a.level[ND + l], tables, pts, r);
+#pragma unroll
+            for (int i = 0; i < L - ND; i++)
+#pragma unroll
+                for (int p = 0; p < P; p++)
+#pragma unroll
+                    for (int k = 0; k < F; k++) {
+                        float& w = x[(p * L + ND + i) * F + k];
+                        w = l == (uint32_t)i ? r[p * F + k] : w;
+                    }
+        });
+    } else if constexpr (ND >= 0) {
+#pragma unroll
+        for (int l = ND; l < L; l++) {
+            float r[P * F];
+            gather_level_f32<P, F, true, false>(a.level[l], tables, pts, r);
+#pragma unroll
+            for (int p = 0; p < P; p++)
+#pragma unroll
+                for (int k = 0; k < F; k++) x[(p * L + l) * F + k] = r[p * F + k];
         }
+    }
 }
 
 // The features of this lane's own segment, every lane of the wave taking part.
-template <int P, int L, int F, int ND>
+template <int P, int L, int F, int ND, Gather G>
 __device__ __forceinline__ void wave_features_f32(const NetArgs& a, const float* __restrict__ tables,
                                                   const float* pts, float* x)
 {
+#pragma unroll
+    for (int k = 0; k < P * L * F; k++) x[k] = 0.f;
     if (__all(in_unit_cube<3 * P>(pts)))
-        gather_features_f32<P, L, F, ND, false>(a, tables, pts, x);
+        gather_features_f32<P, L, F, ND, false, G>(a, tables, pts, x);
     else
-        gather_features_f32<P, L, F, ND, true>(a, tables, pts, x);
+        gather_features_f32<P, L, F, ND, true, G>(a, tables, pts, x);
+}
+
+// WIDE gather of the wave's first `slots` slots (every lane takes part): round by round, lane =
+// level * S + slot of S slots; then each of those slots' lanes collects its levels.
+template <int P, int L, int F>
+__device__ __forceinline__ void gather_wide_f32(const NetArgs& a, const float* __restrict__ tables, uint32_t slots,
+                                                const float* pts, float* x)
+{
+    static_assert(64 % L == 0, "whole levels per wave");
+    constexpr int S = 64 / L < 16 ? 64 / L : 16;
+    const uint32_t lane = threadIdx.x & 63u;
+    const GridLevel lv = a.level[lane / S < (uint32_t)L ? lane / S : 0];
+#pragma unroll
+    for (int k = 0; k < P * L * F; k++) x[k] = 0.f;
+    for (uint32_t r = 0; r < slots; r += S) {
+        float pt[3 * P], f[P * F];
+#pragma unroll
+        for (int c = 0; c < 3 * P; c++) pt[c] = __shfl(pts[c], (int)(r + lane % S));
+        if (__all(in_unit_cube<3 * P>(pt)))
+            gather_level_f32<P, F, false, false>(lv, tables, pt, f);
+        else
+            gather_level_f32<P, F, false, true>(lv, tables, pt, f);
+        const bool mine = lane - r < (uint32_t)S;
+#pragma unroll
+        for (int p = 0; p < P; p++)
+#pragma unroll
+            for (int l = 0; l < L; l++)
+#pragma unroll
+                for (int k = 0; k < F; k++) {
+                    const float v = __shfl(f[p * F + k], (int)(l * S + lane % S));
+                    float& w = x[(p * L + l) * F + k];
+                    w = mine ? v : w;
+                }
+    }
 }
 
 // Own features -> B operands of layer 1: x[2s] serves segments 0..31, x[2s + 1] segments 32..63.
@@ -131,67 +185,70 @@ __device__ __forceinline__ void features_to_b_f32(float* x)
     }
 }
 
-__device__ __forceinline__ void zero_acc(floatx16_t acc[2][2])
+template <int CB>
+__device__ __forceinline__ void zero_acc(floatx16_t acc[2][CB])
 {
 #pragma unroll
     for (int rb = 0; rb < 2; rb++)
 #pragma unroll
-        for (int cb = 0; cb < 2; cb++)
+        for (int cb = 0; cb < CB; cb++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[rb][cb][r] = 0.f;
 }
 
 // acc[rb][cb] += (row block rb of the S k-steps' weights) x (segment block cb): b[2 s + cb].
-template <int S>
-__device__ __forceinline__ void layer_f32(const float2* w, uint32_t lane, const float* b, floatx16_t acc[2][2])
+template <int S, int CB>
+__device__ __forceinline__ void layer_f32(const float2* w, uint32_t lane, const float* b, floatx16_t acc[2][CB])
 {
 #pragma unroll
     for (int s = 0; s < S; s += 2) {
         const float2 w0 = w[(s / 2) * 64 + lane], w1 = w[(S / 2 + s / 2) * 64 + lane];
 #pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const float wa = e ? w0.y : w0.x, wb = e ? w1.y : w1.x;
-            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(wa, b[2 * (s + e)], acc[0][0], 0, 0, 0);
-            acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(wa, b[2 * (s + e) + 1], acc[0][1], 0, 0, 0);
-            acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(wb, b[2 * (s + e)], acc[1][0], 0, 0, 0);
-            acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(wb, b[2 * (s + e) + 1], acc[1][1], 0, 0, 0);
-        }
+        for (int e = 0; e < 2; e++)
+#pragma unroll
+            for (int rb = 0; rb < 2; rb++)
+#pragma unroll
+                for (int cb = 0; cb < CB; cb++) {
+                    const float wa = rb == 0 ? (e ? w0.y : w0.x) : (e ? w1.y : w1.x);
+                    acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(wa, b[2 * (s + e) + cb], acc[rb][cb], 0, 0, 0);
+                }
     }
 }
 
-__device__ __forceinline__ void relu_to_b_f32(const floatx16_t acc[2][2], float b[64])
+template <int CB>
+__device__ __forceinline__ void relu_to_b_f32(const floatx16_t acc[2][CB], float b[64])
 {
 #pragma unroll
     for (int s = 0; s < 32; s++)
 #pragma unroll
-        for (int cb = 0; cb < 2; cb++) {
+        for (int cb = 0; cb < CB; cb++) {
             const float v = acc[s / 16][cb][s % 16];
             b[2 * s + cb] = v > 0.f ? v : 0.f;
         }
 }
 
-// The MLP of the 64 segments of a wave. x[K0]: this lane's own features (overwritten); w: the
-// weight fragments in LDS; z[8]: this lane's logits.
-template <int K0>
+// The MLP of the first 32 * CB segments of a wave. x[K0]: this lane's own features (overwritten);
+// w: the weight fragments in LDS; z[8]: this lane's logits.
+template <int K0, int CB>
 __device__ __forceinline__ void mlp_wave_f32(const float* w, float* x, float z[8])
 {
     typedef F32Layout<K0> Y;
     const uint32_t lane = threadIdx.x & 63u, g = lane >> 5;
     features_to_b_f32<K0>(x);
-    floatx16_t acc[2][2];
-    zero_acc(acc);
-    layer_f32<Y::S1>(reinterpret_cast<const float2*>(w), lane, x, acc);
+    floatx16_t acc[2][CB];
+    zero_acc<CB>(acc);
+    layer_f32<Y::S1, CB>(reinterpret_cast<const float2*>(w), lane, x, acc);
     float b[64];
 #pragma unroll
     for (int layer = 0; layer < 3; layer++) {
-        relu_to_b_f32(acc, b);
-        zero_acc(acc);
-        layer_f32<32>(reinterpret_cast<const float2*>(w + Y::HID) + layer * 2048, lane, b, acc);
+        relu_to_b_f32<CB>(acc, b);
+        zero_acc<CB>(acc);
+        layer_f32<32, CB>(reinterpret_cast<const float2*>(w + Y::HID) + layer * 2048, lane, b, acc);
     }
-    relu_to_b_f32(acc, b);
-    floatx16_t out[2];
+    relu_to_b_f32<CB>(acc, b);
+    floatx16_t out[2] = {};
 #pragma unroll
-    for (int cb = 0; cb < 2; cb++)
+    for (int cb = 0; cb < CB; cb++)
 #pragma unroll
         for (int r = 0; r < 16; r++) out[cb][r] = 0.f;
     const float2* wo = reinterpret_cast<const float2*>(w + Y::OUT);
@@ -201,7 +258,7 @@ __device__ __forceinline__ void mlp_wave_f32(const float* w, float* x, float z[8
 #pragma unroll
         for (int e = 0; e < 2; e++)
 #pragma unroll
-            for (int cb = 0; cb < 2; cb++)
+            for (int cb = 0; cb < CB; cb++)
                 out[cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(e ? v.y : v.x, b[2 * (s + e) + cb], out[cb], 0, 0, 0);
     }
     // Rows 0..3 of a segment block sit in lanes 0..31, rows 4..7 in lanes 32..63.

@@ -237,15 +237,30 @@ struct RayQueue {
     }
 };
 
-// Slots a wave of a persistent launch fills: all 64 once the rays would fill them, else the rays
-// spread evenly over the launch's waves (at least kMinWaveSlots each), so that a small batch uses
-// every CU's L1 and miss queue instead of a few. The count may live on the device, so the kernel
-// decides; the host sizes the grid (query_blocks, kernels/launch.h).
-__device__ __forceinline__ uint32_t wave_slots(uint32_t n_rays)
+// First rays of a wave. Static launches (a.static_slots > 0: every ray has a slot) hand ray
+// wave * slots + lane to each lane and never touch the queue; the others start with empty slots
+// and claim. A queued batch whose count (which may live on the device) would give every wave 8
+// rays or fewer is spread evenly over all waves: few rays per wave then answer sooner than full
+// waves on a few CUs (4,096 rays 168 against 234 us); beyond that full waves are better (65,536
+// rays 256 us with 64 rays per wave, 297 us with 32). Returns the slots in use.
+template <bool PARTS>
+__device__ __forceinline__ uint32_t first_rays(const NetArgs& a, const RayBatch& b, RayQueue& q, Slot& s)
 {
-    const uint32_t waves = gridDim.x * (blockDim.x >> 6);
-    const uint32_t even  = n_rays / waves + (n_rays % waves != 0u ? 1u : 0u);
-    return even < kMinWaveSlots ? kMinWaveSlots : (even < 64u ? even : 64u);
+    const uint32_t lane = threadIdx.x & 63u, per_block = blockDim.x >> 6, waves = gridDim.x * per_block;
+    if (a.static_slots != 0u) {
+        const uint32_t i = (blockIdx.x * per_block + (threadIdx.x >> 6)) * a.static_slots + lane;
+        s.state = SLOT_DONE;
+        if (lane < a.static_slots && i < q.n_rays) {
+            s.state = SLOT_NEW;
+            batch_locate<PARTS>(b, batch_ray(b, q.ray_of(i)), s.part, s.ray_id);
+        }
+        q.tried = q.bands;  // nothing left to claim
+        return a.static_slots;
+    }
+    const uint32_t even  = q.n_rays / waves + (q.n_rays % waves != 0u ? 1u : 0u);
+    const uint32_t slots = even > 8u ? 64u : (even > 4u ? even : 4u);
+    s.state = lane < slots ? SLOT_EMPTY : SLOT_DONE;
+    return slots;
 }
 
 // Phase A. Returns false when the wave has no segment left to evaluate (all slots DONE).

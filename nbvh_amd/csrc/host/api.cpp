@@ -412,7 +412,6 @@ void run_query_ordered(nbvh_ctx* ctx, const nbvh_scene* s, const nbvh_query_para
         lease = own.get();
     }
     uint32_t* counter = fixed_counters ? fixed_counters : lease->counters();
-    hip_check(zero_u32(counter, nbvh_ctx::kCounterWords, stream), "counter reset");
     bool supported = false;
     if (p->precision == NBVH_PREC_FP32)
         hip_check(query_fp32(a, batch, counter, (uint32_t)ctx->n_cus, stream, &supported), "fp32 query");

@@ -17,7 +17,7 @@ namespace dev {
 // inputs); with the waves' stacks (48 KB) and the node cache (16 KB) it takes 138 of 160 KB.
 constexpr int kF32Waves = 8;
 
-template <int P, int L, int F, bool PARTS, int ND>
+template <int P, int L, int F, bool PARTS, int ND, Gather G>
 __global__ __launch_bounds__(64 * kF32Waves, 2) void neural_query_fp32_kernel(NetArgs a, RayBatch b,
                                                                              uint32_t* __restrict__ queue)
 {
@@ -34,19 +34,26 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void neural_query_fp32_kernel(Ne
     RayQueue q;
     q.init(queue, batch_count(b), a.image_width, a.queue_bands);
     Slot s;
-    s.state = lane < wave_slots(q.n_rays) ? SLOT_EMPTY : SLOT_DONE;
+    const uint32_t slots = first_rays<PARTS>(a, b, q, s);
     while (fill_slots<PARTS>(a, nodes, s, st, b, q)) {
         float x[K0];
-        if (s.state == SLOT_SEG) {
+        if constexpr (G == Gather::WIDE) {
+            float pts[3 * P];
+#pragma unroll
+            for (int c = 0; c < 3 * P; c++) pts[c] = 0.5f;
+            if (s.state == SLOT_SEG) encode_segment(a, s.ray, s.seg_mint, s.seg_maxt, pts, &s.rng);
+            gather_wide_f32<P, L, F>(a, a.tables_f32, slots, pts, x);
+        } else if (s.state == SLOT_SEG) {
             float pts[3 * P];
             encode_segment(a, s.ray, s.seg_mint, s.seg_maxt, pts, &s.rng);
-            wave_features_f32<P, L, F, ND>(a, a.tables_f32, pts, x);
+            wave_features_f32<P, L, F, ND, G>(a, a.tables_f32, pts, x);
         } else {
 #pragma unroll
             for (int k = 0; k < K0; k++) x[k] = 0.f;
         }
+        // WIDE: at most 16 slots, the second block of 32 segments is empty.
         float z[8];
-        mlp_wave_f32<K0>(reinterpret_cast<const float*>(w_lds), x, z);
+        mlp_wave_f32<K0, G == Gather::WIDE ? 1 : 2>(reinterpret_cast<const float*>(w_lds), x, z);
         if (s.state == SLOT_SEG) consume_segment<PARTS>(a, s, z, b);
     }
 }
@@ -71,13 +78,13 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void network_fp32_kernel(NetArgs
             float pts[3 * P];
 #pragma unroll
             for (int c = 0; c < 3 * P; c++) pts[c] = in[(size_t)i * (3 * P) + c];
-            wave_features_f32<P, L, F, ND>(a, a.tables_f32, pts, x);
+            wave_features_f32<P, L, F, ND, Gather::LEVELS>(a, a.tables_f32, pts, x);
         } else {
 #pragma unroll
             for (int k = 0; k < K0; k++) x[k] = 0.f;
         }
         float z[8];
-        mlp_wave_f32<K0>(reinterpret_cast<const float*>(w_lds), x, z);
+        mlp_wave_f32<K0, 2>(reinterpret_cast<const float*>(w_lds), x, z);
         if (i < n) {
 #pragma unroll
             for (int j = 0; j < 8; j++) {
@@ -90,32 +97,40 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void network_fp32_kernel(NetArgs
 
 }  // namespace dev
 
-template <int P, int L, int F, bool PARTS, int ND>
+template <int P, int L, int F, bool PARTS>
 static hipError_t launch_fp32_query_k(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus,
                                       hipStream_t stream)
 {
-    auto k = dev::neural_query_fp32_kernel<P, L, F, PARTS, ND>;
+    using dev::Gather;
     constexpr uint32_t threads = 64 * dev::kF32Waves;
+    auto k = dev::neural_query_fp32_kernel<P, L, F, PARTS, -1, Gather::LEVELS>;
     static const uint32_t bpc = blocks_per_cu(k, threads);
     const uint32_t cap = a.blocks_per_cu != 0u && a.blocks_per_cu < bpc ? a.blocks_per_cu : bpc;
-    const uint32_t blocks = query_blocks(rb.n, dev::kF32Waves, n_cus * cap);
-    hipLaunchKernelGGL(k, dim3(blocks), dim3(threads), 0, stream, a, rb, queue);
+    const QueryGrid g = query_grid(rb, dev::kF32Waves, n_cus * cap, 64u / L < 16u ? 64u / L : 16u);
+    NetArgs args = a;
+    args.static_slots = g.static_slots;
+    if (g.static_slots == 0u) {
+        const hipError_t e = zero_u32(queue, dev::kQueueWords, stream);
+        if (e != hipSuccess) return e;
+    }
+    if (g.wide) {
+        k = dev::neural_query_fp32_kernel<P, L, F, PARTS, -1, Gather::WIDE>;
+    } else if constexpr (L > kDensePrefix) {
+        // The hash-only gather for grids whose levels from the 4th on are hashed (the two
+        // benchmark shapes); other grids take the general gather.
+        if (a.n_dense == (uint32_t)kDensePrefix)
+            k = dev::neural_query_fp32_kernel<P, L, F, PARTS, kDensePrefix, dev::kQueryGather<L, kDensePrefix>>;
+    }
+    hipLaunchKernelGGL(k, dim3(g.blocks), dim3(threads), 0, stream, args, rb, queue);
     return hipGetLastError();
 }
 
-// The hash-only gather for grids whose levels from the 4th on are hashed (the two benchmark
-// shapes); other grids take the general gather.
 template <int P, int L, int F>
 static hipError_t launch_fp32_query(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus,
                                     hipStream_t stream)
 {
-    if constexpr (L > kDensePrefix) {
-        if (a.n_dense == (uint32_t)kDensePrefix)
-            return rb.parts ? launch_fp32_query_k<P, L, F, true, kDensePrefix>(a, rb, queue, n_cus, stream)
-                            : launch_fp32_query_k<P, L, F, false, kDensePrefix>(a, rb, queue, n_cus, stream);
-    }
-    return rb.parts ? launch_fp32_query_k<P, L, F, true, -1>(a, rb, queue, n_cus, stream)
-                    : launch_fp32_query_k<P, L, F, false, -1>(a, rb, queue, n_cus, stream);
+    return rb.parts ? launch_fp32_query_k<P, L, F, true>(a, rb, queue, n_cus, stream)
+                    : launch_fp32_query_k<P, L, F, false>(a, rb, queue, n_cus, stream);
 }
 
 template <int P, int L, int F, int ND>

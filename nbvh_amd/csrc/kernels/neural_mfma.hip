@@ -67,31 +67,17 @@ __device__ __forceinline__ void swap_halves(V& x, V& y)
     y = __builtin_bit_cast(V, b);
 }
 
-// Cache policy (buffer-load aux bits: 1 sc0, 2 nt) of the corner gathers of levels
-// >= NBVH_GATHER_POLICY_FROM; the coarser levels use the default policy.
-#ifndef NBVH_GATHER_POLICY_FROM
-#define NBVH_GATHER_POLICY_FROM 64
-#endif
-#ifndef NBVH_GATHER_POLICY
-#define NBVH_GATHER_POLICY 0
-#endif
-
-template <int F, int AUX>
+template <int F>
 __device__ __forceinline__ void load_corner(__amdgpu_buffer_rsrc_t tab, uint32_t off, uint32_t q[F / 2])
 {
     if constexpr (F == 2) {
-        q[0] = __builtin_amdgcn_raw_buffer_load_b32(tab, off, 0, AUX);
+        q[0] = __builtin_amdgcn_raw_buffer_load_b32(tab, off, 0, 0);
     } else {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b64(tab, off, 0, AUX);
+        const auto v = __builtin_amdgcn_raw_buffer_load_b64(tab, off, 0, 0);
         q[0] = v[0];
         q[1] = v[1];
     }
 }
-
-// Levels whose gathers are issued together (G x 8 loads in flight per lane before the first use).
-#ifndef NBVH_GATHER_GROUP
-#define NBVH_GATHER_GROUP 4
-#endif
 
 // Layer-1 B operands. Every lane computes all K0 features of its own segment (wave-uniform
 // gather code); lo[s] holds features 8s..8s+7, hi[s] features K0/2+8s..K0/2+8s+7. Column block 0
@@ -119,36 +105,32 @@ __device__ __forceinline__ void level_offsets(const GridLevel& lv, float x, floa
     for (int c = 0; c < 8; c++) off[c] = (idx[c] + lv.offset) << kShift;
 }
 
-// One group of G levels of point p: all 8G corner offsets, then all 8G loads, then the corner
-// weights and the FP32 accumulation over corners 0..7 (tcnn's trilinear weights); the features
-// go to the layer-1 operand halves lo / hi as 16-bit values.
-template <int P, int L, int F, int G, bool BF16, bool HASHED, bool EXACT>
-__device__ __forceinline__ void gather_group(const NetArgs& a, __amdgpu_buffer_rsrc_t tab, const float* pt, int p,
-                                             int l0, typename Frag<BF16>::vec* lo, typename Frag<BF16>::vec* hi)
+// One level, all P points: the 8 P corner offsets, then all loads, then the corner weights and the
+// FP32 accumulation over corners 0..7 (tcnn's trilinear weights). out[p * F / 2 ..]: the level's
+// features of point p as 16-bit pairs.
+template <int P, int F, bool BF16, bool HASHED, bool EXACT>
+__device__ __forceinline__ void gather_level(const GridLevel& lv, __amdgpu_buffer_rsrc_t tab, const float* pts,
+                                             uint32_t* out)
 {
-    constexpr int HALF = P * L * F / 2;
     typedef typename Frag<BF16>::elem E;
-    uint32_t off[G][8];
-    float fr[G][3];
+    typedef E pair_t __attribute__((ext_vector_type(2)));
+    uint32_t off[P][8];
+    float fr[P][3];
 #pragma unroll
-    for (int i = 0; i < G; i++) level_offsets<F, HASHED, EXACT>(a.level[l0 + i], pt[0], pt[1], pt[2], off[i], fr[i]);
+    for (int p = 0; p < P; p++)
+        level_offsets<F, HASHED, EXACT>(lv, pts[3 * p], pts[3 * p + 1], pts[3 * p + 2], off[p], fr[p]);
     // One load per corner. (Measured: serving x-neighbour corners with one 16-byte load plus a
     // range-masked second load halves the throughput, so corners stay separate.)
-    uint32_t q[G][8][F / 2];
+    uint32_t q[P][8][F / 2];
 #pragma unroll
-    for (int i = 0; i < G; i++)
+    for (int p = 0; p < P; p++)
 #pragma unroll
-        for (int c = 0; c < 8; c++) {
-            if (l0 + i >= NBVH_GATHER_POLICY_FROM)
-                load_corner<F, NBVH_GATHER_POLICY>(tab, off[i][c], q[i][c]);
-            else
-                load_corner<F, 0>(tab, off[i][c], q[i][c]);
-        }
+        for (int c = 0; c < 8; c++) load_corner<F>(tab, off[p][c], q[p][c]);
 #pragma unroll
-    for (int i = 0; i < G; i++) {
+    for (int p = 0; p < P; p++) {
         // tcnn's corner weights ((1 * w_x) * w_y) * w_z, the x-y products shared by the z pair.
-        const float wx[2] = {1.f - fr[i][0], fr[i][0]}, wy[2] = {1.f - fr[i][1], fr[i][1]};
-        const float wz[2] = {1.f - fr[i][2], fr[i][2]};
+        const float wx[2] = {1.f - fr[p][0], fr[p][0]}, wy[2] = {1.f - fr[p][1], fr[p][1]};
+        const float wz[2] = {1.f - fr[p][2], fr[p][2]};
         float acc[F];
 #pragma unroll
         for (int k = 0; k < F; k++) acc[k] = 0.f;
@@ -157,57 +139,124 @@ __device__ __forceinline__ void gather_group(const NetArgs& a, __amdgpu_buffer_r
             const float w = trilinear_weight(c, wx, wy, wz);
 #pragma unroll
             for (int k = 0; k < F; k++) {
-                const uint32_t bits = (k & 1) ? (q[i][c][k / 2] >> 16) : (q[i][c][k / 2] & 0xFFFFu);
+                const uint32_t bits = (k & 1) ? (q[p][c][k / 2] >> 16) : (q[p][c][k / 2] & 0xFFFFu);
                 acc[k] = fmaf(w, half_bits_to_float(bits), acc[k]);
             }
         }
 #pragma unroll
-        for (int f = 0; f < F; f++) {
-            const int k = p * L * F + (l0 + i) * F + f;
-            if (k < HALF)
-                lo[k / 8][k % 8] = (E)acc[f];
-            else
-                hi[(k - HALF) / 8][(k - HALF) % 8] = (E)acc[f];
+        for (int j = 0; j < F / 2; j++) {
+            const pair_t v = {(E)acc[2 * j], (E)acc[2 * j + 1]};
+            out[p * (F / 2) + j] = __builtin_bit_cast(uint32_t, v);
         }
     }
 }
 
+// All features of the lane's segment, pair j of feature k = 2j, 2j + 1 (k = p * L * F + l * F + f).
 // ND >= 0: the kernel is specialised for grids whose levels [ND, L) are hashed (n_dense == ND,
-// checked at launch); groups of those levels take the hash-only form, the others the general
-// form. ND < 0: every level takes the general form (any grid). EXACT: the full modulo for
-// points outside the unit cube (dense levels only; the hash is exact everywhere).
-template <int P, int L, int F, bool BF16, bool EXACT, int ND>
+// checked at launch): those levels take the hash-only form, the others the general form. ND < 0:
+// every level takes the general form (any grid). EXACT: the full modulo for points outside the
+// unit cube (dense levels only; the hash is exact everywhere).
+template <int P, int L, int F, bool BF16, bool EXACT, int ND, Gather G>
 __device__ __forceinline__ void gather_operands(const NetArgs& a, __amdgpu_buffer_rsrc_t tab, const float* pts,
-                                                typename Frag<BF16>::vec* lo, typename Frag<BF16>::vec* hi)
+                                                uint32_t* x)
 {
-    constexpr int G = (L % NBVH_GATHER_GROUP == 0) ? NBVH_GATHER_GROUP : 1;
     static_assert(F == 2 || F == 4, "FP16 gather implemented for F = 2 and F = 4");
+    constexpr int H = F / 2;  // 16-bit pairs per level and point
 #pragma unroll
-    for (int p = 0; p < P; p++) {
+    for (int l = 0; l < (ND >= 0 ? ND : L); l++) {
+        uint32_t r[P * H];
+        gather_level<P, F, BF16, false, EXACT>(a.level[l], tab, pts, r);
 #pragma unroll
-        for (int l0 = 0; l0 < L; l0 += G) {
-            if (ND >= 0 && l0 >= ND)  // folded at compile time after unrolling
-                gather_group<P, L, F, G, BF16, true, false>(a, tab, pts + 3 * p, p, l0, lo, hi);
-            else
-                gather_group<P, L, F, G, BF16, false, EXACT>(a, tab, pts + 3 * p, p, l0, lo, hi);
+        for (int p = 0; p < P; p++)
+#pragma unroll
+            for (int j = 0; j < H; j++) x[(p * L + l) * H + j] = r[p * H + j];
+    }
+    if constexpr (ND >= 0) {
+        if constexpr (G == Gather::PHASES) {
+            level_phases<L - ND>([&](uint32_t l) {
+                uint32_t r[P * H];
+                gather_level<P, F, BF16, true, false>(a.level[ND + l], tab, pts, r);
+#pragma unroll
+                for (int i = 0; i < L - ND; i++)
+#pragma unroll
+                    for (int p = 0; p < P; p++)
+#pragma unroll
+                        for (int j = 0; j < H; j++) {
+                            uint32_t& w = x[(p * L + ND + i) * H + j];
+                            w = l == (uint32_t)i ? r[p * H + j] : w;
+                        }
+            });
+        } else {
+#pragma unroll
+            for (int l = ND; l < L; l++) {
+                uint32_t r[P * H];
+                gather_level<P, F, BF16, true, false>(a.level[l], tab, pts, r);
+#pragma unroll
+                for (int p = 0; p < P; p++)
+#pragma unroll
+                    for (int j = 0; j < H; j++) x[(p * L + l) * H + j] = r[p * H + j];
+            }
         }
     }
 }
 
-template <int P, int L, int F, bool BF16, int ND>
-__device__ __forceinline__ void layer1_operands(const NetArgs& a, const float* pts,
+// WIDE gather of the wave's first `slots` slots: round by round, lane = level * S + slot of 64 / L
+// slots; then each of those slots' lanes collects its levels (one ds_bpermute per 16-bit pair).
+template <int P, int L, int F, bool BF16>
+__device__ __forceinline__ void gather_wide(const NetArgs& a, __amdgpu_buffer_rsrc_t tab, uint32_t slots,
+                                            const float* pts, uint32_t* x)
+{
+    static_assert(64 % L == 0, "whole levels per wave");
+    constexpr int S = 64 / L, H = F / 2;
+    const uint32_t lane = threadIdx.x & 63u;
+    const GridLevel lv = a.level[lane / S];
+    for (uint32_t r = 0; r < slots; r += S) {
+        float pt[3 * P];
+#pragma unroll
+        for (int c = 0; c < 3 * P; c++) pt[c] = __shfl(pts[c], (int)(r + lane % S));
+        uint32_t f[P * H];
+        if (__all(in_unit_cube<3 * P>(pt)))
+            gather_level<P, F, BF16, false, false>(lv, tab, pt, f);
+        else
+            gather_level<P, F, BF16, false, true>(lv, tab, pt, f);
+        const bool mine = lane - r < (uint32_t)S;
+#pragma unroll
+        for (int p = 0; p < P; p++)
+#pragma unroll
+            for (int l = 0; l < L; l++)
+#pragma unroll
+                for (int j = 0; j < H; j++) {
+                    const uint32_t v = (uint32_t)__shfl((int)f[p * H + j], (int)(l * S + lane % S));
+                    uint32_t& w = x[(p * L + l) * H + j];
+                    w = mine ? v : w;
+                }
+    }
+}
+
+template <int P, int L, int F, bool BF16, int ND, Gather G>
+__device__ __forceinline__ void layer1_operands(const NetArgs& a, uint32_t slots, const float* pts,
                                                 typename Frag<BF16>::vec lo[P * L * F / 16],
                                                 typename Frag<BF16>::vec hi[P * L * F / 16])
 {
     constexpr int K0 = P * L * F;
+    typedef typename Frag<BF16>::vec V;
     const __amdgpu_buffer_rsrc_t tab =
         __builtin_amdgcn_make_buffer_rsrc((void*)a.tables_f16, (short)0, (int)a.tables_f16_bytes, 0x00020000);
-    if (__all(in_unit_cube<3 * P>(pts)))
-        gather_operands<P, L, F, BF16, false, ND>(a, tab, pts, lo, hi);
-    else
-        gather_operands<P, L, F, BF16, true, ND>(a, tab, pts, lo, hi);
+    uint32_t x[K0 / 2] = {};
+    if constexpr (G == Gather::WIDE) {
+        gather_wide<P, L, F, BF16>(a, tab, slots, pts, x);
+    } else if (__all(in_unit_cube<3 * P>(pts))) {
+        gather_operands<P, L, F, BF16, false, ND, G>(a, tab, pts, x);
+    } else {
+        gather_operands<P, L, F, BF16, true, ND, G>(a, tab, pts, x);
+    }
 #pragma unroll
-    for (int s = 0; s < K0 / 16; s++) swap_halves(lo[s], hi[s]);
+    for (int s = 0; s < K0 / 16; s++) {
+        lo[s] = __builtin_bit_cast(V, make_uint4(x[4 * s], x[4 * s + 1], x[4 * s + 2], x[4 * s + 3]));
+        const int h = K0 / 4 + 4 * s;
+        hi[s] = __builtin_bit_cast(V, make_uint4(x[h], x[h + 1], x[h + 2], x[h + 3]));
+        swap_halves(lo[s], hi[s]);
+    }
 }
 
 // The 8 output rows of this lane's own segment (column lane%32 of column block g), times inv.
@@ -245,9 +294,9 @@ __device__ __forceinline__ void acc_to_b(const floatx16 acc[2][2], typename Frag
 
 // The whole network for the 64 segments of a wave. own[3P]: this lane's segment points.
 // Returns this lane's 8 logits (descaled). wfrag: LDS fragments (16 B per lane each).
-template <int P, int L, int F, bool BF16, int ND>
-__device__ __forceinline__ void mfma_network(const NetArgs& a, const uint4* __restrict__ wfrag, const float* own,
-                                             float z[8])
+template <int P, int L, int F, bool BF16, int ND, Gather G>
+__device__ __forceinline__ void mfma_network(const NetArgs& a, const uint4* __restrict__ wfrag, uint32_t slots,
+                                             const float* own, float z[8])
 {
     constexpr int K0 = P * L * F;
     typedef MlpShape<K0> S;
@@ -256,7 +305,7 @@ __device__ __forceinline__ void mfma_network(const NetArgs& a, const uint4* __re
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t g    = lane >> 5;
     V b1[2][S::KS1];
-    layer1_operands<P, L, F, BF16, ND>(a, own, b1[0], b1[1]);
+    layer1_operands<P, L, F, BF16, ND, G>(a, slots, own, b1[0], b1[1]);
     floatx16 acc[2][2];
 #pragma unroll
     for (int rb = 0; rb < 2; rb++)
@@ -311,12 +360,34 @@ __device__ __forceinline__ void mfma_network(const NetArgs& a, const uint4* __re
     gather_logits(out, g, a.inv_table_scale, z);
 }
 
+// Waves per workgroup of the query kernel; the workgroup shares one LDS copy of the weights.
+#ifndef NBVH_MFMA_BLOCK_WAVES
+#define NBVH_MFMA_BLOCK_WAVES 4
+#endif
+constexpr int kWavesPerBlock = NBVH_MFMA_BLOCK_WAVES;
+
+// N elements from global memory into LDS by the whole workgroup: a fixed trip count, so that all
+// of a thread's loads are in flight before the first store.
+template <int N, typename T>
+__device__ __forceinline__ void stage(const T* __restrict__ src, T* lds)
+{
+    constexpr int B = 64 * kWavesPerBlock;
+    constexpr int FULL = N / B;
+    const int t = (int)threadIdx.x;
+    T v[FULL > 0 ? FULL : 1];
+#pragma unroll
+    for (int i = 0; i < FULL; i++) v[i] = src[i * B + t];
+#pragma unroll
+    for (int i = 0; i < FULL; i++) lds[i * B + t] = v[i];
+    if (N % B != 0 && FULL * B + t < N) lds[FULL * B + t] = src[FULL * B + t];
+}
+
 template <int P, int L, int F, bool BF16>
 __device__ __forceinline__ void stage_weights(const NetArgs& a, uint4* wfrag)
 {
     constexpr int NF = MlpShape<P * L * F>::N_FRAG;
     const uint4* src = reinterpret_cast<const uint4*>(a.mlp_frag) + (BF16 ? (size_t)NF * 64 : 0);
-    for (uint32_t i = threadIdx.x; i < (uint32_t)NF * 64; i += blockDim.x) wfrag[i] = src[i];
+    stage<NF * 64>(src, wfrag);
     __syncthreads();
 }
 
@@ -385,16 +456,15 @@ __device__ __forceinline__ void stage_weights_fp8(const NetArgs& a, Fp8Lds<K0>& 
     typedef MlpShape<K0> S;
     const uint4* f16 = reinterpret_cast<const uint4*>(a.mlp_frag);
     const uint2* f8  = reinterpret_cast<const uint2*>(a.mlp_frag_fp8);
-    for (uint32_t i = threadIdx.x; i < (uint32_t)S::F_L1 * 64; i += blockDim.x) w.l1[i] = f16[i];
-    for (uint32_t i = threadIdx.x; i < 4u * 64; i += blockDim.x) w.out[i] = f16[(size_t)(S::F_L1 + 3 * S::F_HID) * 64 + i];
-    for (uint32_t i = threadIdx.x; i < (uint32_t)Fp8Weights::kHidden * Fp8Weights::kFragsPerLayer * 64; i += blockDim.x)
-        w.hid[i] = f8[i];
+    stage<S::F_L1 * 64>(f16, w.l1);
+    stage<4 * 64>(f16 + (size_t)(S::F_L1 + 3 * S::F_HID) * 64, w.out);
+    stage<Fp8Weights::kHidden * Fp8Weights::kFragsPerLayer * 64>(f8, w.hid);
     __syncthreads();
 }
 
-template <int P, int L, int F, int ND>
-__device__ __forceinline__ void mfma_network_fp8(const NetArgs& a, const Fp8Lds<P * L * F>& w, const float* own,
-                                                 float z[8])
+template <int P, int L, int F, int ND, Gather G>
+__device__ __forceinline__ void mfma_network_fp8(const NetArgs& a, const Fp8Lds<P * L * F>& w, uint32_t slots,
+                                                 const float* own, float z[8])
 {
     constexpr int K0 = P * L * F;
     typedef MlpShape<K0> S;
@@ -404,7 +474,7 @@ __device__ __forceinline__ void mfma_network_fp8(const NetArgs& a, const Fp8Lds<
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t g    = lane >> 5;
     V b1[2][S::KS1];
-    layer1_operands<P, L, F, false, ND>(a, own, b1[0], b1[1]);
+    layer1_operands<P, L, F, false, ND, G>(a, slots, own, b1[0], b1[1]);
     floatx16 acc[2][2];
 #pragma unroll
     for (int rb = 0; rb < 2; rb++)
@@ -481,17 +551,12 @@ __device__ __forceinline__ void mfma_network_fp8(const NetArgs& a, const Fp8Lds<
     gather_logits(out, g, 1.f / cum[g], z);
 }
 
-// Waves per workgroup of the query kernel; the workgroup shares one LDS copy of the weights.
-#ifndef NBVH_MFMA_BLOCK_WAVES
-#define NBVH_MFMA_BLOCK_WAVES 4
-#endif
-constexpr int kWavesPerBlock = NBVH_MFMA_BLOCK_WAVES;
 // Minimum waves per SIMD the register allocation must allow (latency hiding of the gathers).
 #ifndef NBVH_MFMA_WAVES_PER_EU
 #define NBVH_MFMA_WAVES_PER_EU 2
 #endif
 
-template <int P, int L, int F, bool BF16, bool PARTS, int ND>
+template <int P, int L, int F, bool BF16, bool PARTS, int ND, Gather G>
 __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void neural_query_mfma_kernel(NetArgs a,
                                                                                 RayBatch b,
                                                                                 uint32_t* __restrict__ queue)
@@ -505,10 +570,10 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void n
     const CachedNodes nodes{a.nodes, node_lds, n_cached};
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     LdsStack st{stack_lds + wave * kNeuralStackSize * 64 + lane, 0};
-    Slot s;
-    s.state = SLOT_EMPTY;
     RayQueue q;
     q.init(queue, batch_count(b), a.image_width, a.queue_bands);
+    Slot s;
+    const uint32_t slots = first_rays<PARTS>(a, b, q, s);
     while (fill_slots<PARTS>(a, nodes, s, st, b, q)) {
         float own[3 * P];
         if (s.state == SLOT_SEG) {
@@ -518,13 +583,13 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void n
             for (int c = 0; c < 3 * P; c++) own[c] = 0.5f;
         }
         float z[8];
-        mfma_network<P, L, F, BF16, ND>(a, wfrag, own, z);
+        mfma_network<P, L, F, BF16, ND, G>(a, wfrag, slots, own, z);
         if (s.state == SLOT_SEG) consume_segment<PARTS>(a, s, z, b);
     }
 }
 
 template <int P, int L, int F, bool BF16, int ND>
-__global__ __launch_bounds__(64 * kWavesPerBlock) void network_mfma_kernel(NetArgs a, const float* __restrict__ in,
+__global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void network_mfma_kernel(NetArgs a, const float* __restrict__ in,
                                                                            uint32_t n, float* __restrict__ out,
                                                                            float* __restrict__ logits)
 {
@@ -534,12 +599,13 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void network_mfma_kernel(NetAr
     // Persistent over chunks of blockDim.x inputs (the chunk start is block-uniform, so every wave
     // takes part in each MFMA); the weights are staged once per resident workgroup.
     for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
+        asm volatile("" ::: "memory");  // keeps the weights' LDS reads in the loop (hoisted: one wave per SIMD)
         const uint32_t i = base + threadIdx.x;
         float own[3 * P];
 #pragma unroll
         for (int c = 0; c < 3 * P; c++) own[c] = i < n ? in[(size_t)i * (3 * P) + c] : 0.5f;
         float z[8];
-        mfma_network<P, L, F, BF16, ND>(a, wfrag, own, z);
+        mfma_network<P, L, F, BF16, ND, Gather::LEVELS>(a, wfrag, 64u, own, z);
         if (i < n) {
 #pragma unroll
             for (int j = 0; j < 8; j++) {
@@ -550,7 +616,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void network_mfma_kernel(NetAr
     }
 }
 
-template <int P, int L, int F, bool PARTS, int ND>
+template <int P, int L, int F, bool PARTS, int ND, Gather G>
 __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void neural_query_fp8_kernel(NetArgs a,
                                                                                RayBatch b,
                                                                                uint32_t* __restrict__ queue)
@@ -563,10 +629,10 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void n
     const CachedNodes nodes{a.nodes, node_lds, n_cached};
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     LdsStack st{stack_lds + wave * kNeuralStackSize * 64 + lane, 0};
-    Slot s;
-    s.state = SLOT_EMPTY;
     RayQueue q;
     q.init(queue, batch_count(b), a.image_width, a.queue_bands);
+    Slot s;
+    const uint32_t slots = first_rays<PARTS>(a, b, q, s);
     while (fill_slots<PARTS>(a, nodes, s, st, b, q)) {
         float own[3 * P];
         if (s.state == SLOT_SEG) {
@@ -576,25 +642,26 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void n
             for (int c = 0; c < 3 * P; c++) own[c] = 0.5f;
         }
         float z[8];
-        mfma_network_fp8<P, L, F, ND>(a, w, own, z);
+        mfma_network_fp8<P, L, F, ND, G>(a, w, slots, own, z);
         if (s.state == SLOT_SEG) consume_segment<PARTS>(a, s, z, b);
     }
 }
 
 template <int P, int L, int F, int ND>
-__global__ __launch_bounds__(64 * kWavesPerBlock) void network_fp8_kernel(NetArgs a, const float* __restrict__ in,
+__global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void network_fp8_kernel(NetArgs a, const float* __restrict__ in,
                                                                           uint32_t n, float* __restrict__ out,
                                                                           float* __restrict__ logits)
 {
     __shared__ Fp8Lds<P * L * F> w;
     stage_weights_fp8<P * L * F>(a, w);
     for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
+        asm volatile("" ::: "memory");  // keeps the weights' LDS reads in the loop (hoisted: one wave per SIMD)
         const uint32_t i = base + threadIdx.x;
         float own[3 * P];
 #pragma unroll
         for (int c = 0; c < 3 * P; c++) own[c] = i < n ? in[(size_t)i * (3 * P) + c] : 0.5f;
         float z[8];
-        mfma_network_fp8<P, L, F, ND>(a, w, own, z);
+        mfma_network_fp8<P, L, F, ND, Gather::LEVELS>(a, w, 64u, own, z);
         if (i < n) {
 #pragma unroll
             for (int j = 0; j < 8; j++) {
@@ -609,31 +676,45 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void network_fp8_kernel(NetArg
 
 namespace {
 
-template <int P, int L, int F, bool BF16, bool PARTS, int ND>
+// PREC: NBVH_PREC_FP16, _BF16 or _FP8.
+template <int P, int L, int F, uint32_t PREC, bool PARTS, int ND, dev::Gather G>
+auto query_kernel()
+{
+    if constexpr (PREC == NBVH_PREC_FP8)
+        return dev::neural_query_fp8_kernel<P, L, F, PARTS, ND, G>;
+    else
+        return dev::neural_query_mfma_kernel<P, L, F, PREC == NBVH_PREC_BF16, PARTS, ND, G>;
+}
+
+template <int P, int L, int F, uint32_t PREC, bool PARTS>
 hipError_t launch_query_k(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus, hipStream_t stream)
 {
-    auto k = dev::neural_query_mfma_kernel<P, L, F, BF16, PARTS, ND>;
-    static const uint32_t bpc = blocks_per_cu(k, 64 * dev::kWavesPerBlock);
-    const uint32_t per_block = 64 * dev::kWavesPerBlock;
-    uint32_t blocks = (rb.n + per_block - 1) / per_block;
+    using dev::Gather;
+    constexpr uint32_t threads = 64 * dev::kWavesPerBlock;
+    constexpr int ND = kDensePrefix;
+    const auto wide  = query_kernel<P, L, F, PREC, PARTS, -1, Gather::WIDE>();
+    const auto dense = query_kernel<P, L, F, PREC, PARTS, ND, dev::kQueryGather<L, ND>>();
+    const auto any   = query_kernel<P, L, F, PREC, PARTS, -1, Gather::LEVELS>();
+    // Every variant is bounded to two waves per SIMD and holds the same LDS.
+    static const uint32_t bpc = blocks_per_cu(any, threads);
     const uint32_t cap = a.blocks_per_cu != 0u && a.blocks_per_cu < bpc ? a.blocks_per_cu : bpc;
-    blocks = blocks < n_cus * cap ? blocks : n_cus * cap;
-    hipLaunchKernelGGL(k, dim3(blocks), dim3(per_block), 0, stream, a, rb, queue);
+    const QueryGrid g = query_grid(rb, dev::kWavesPerBlock, n_cus * cap, 64u / L);
+    NetArgs args = a;
+    args.static_slots = g.static_slots;
+    if (g.static_slots == 0u) {
+        const hipError_t e = zero_u32(queue, dev::kQueueWords, stream);
+        if (e != hipSuccess) return e;
+    }
+    const auto k = g.wide ? wide : a.n_dense == (uint32_t)ND ? dense : any;
+    hipLaunchKernelGGL(k, dim3(g.blocks), dim3(threads), 0, stream, args, rb, queue);
     return hipGetLastError();
 }
 
-template <int P, int L, int F, bool BF16, int ND>
-hipError_t launch_query_nd(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus, hipStream_t stream)
-{
-    return rb.parts ? launch_query_k<P, L, F, BF16, true, ND>(a, rb, queue, n_cus, stream)
-                    : launch_query_k<P, L, F, BF16, false, ND>(a, rb, queue, n_cus, stream);
-}
-
-template <int P, int L, int F, bool BF16>
+template <int P, int L, int F, uint32_t PREC>
 hipError_t launch_query(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus, hipStream_t stream)
 {
-    return a.n_dense == (uint32_t)kDensePrefix ? launch_query_nd<P, L, F, BF16, kDensePrefix>(a, rb, queue, n_cus, stream)
-                                               : launch_query_nd<P, L, F, BF16, -1>(a, rb, queue, n_cus, stream);
+    return rb.parts ? launch_query_k<P, L, F, PREC, true>(a, rb, queue, n_cus, stream)
+                    : launch_query_k<P, L, F, PREC, false>(a, rb, queue, n_cus, stream);
 }
 
 template <int P, int L, int F, bool BF16, int ND>
@@ -656,35 +737,6 @@ hipError_t launch_network(const NetArgs& a, const float* in, uint32_t n, float* 
     return a.n_dense == (uint32_t)kDensePrefix
                ? launch_network_nd<P, L, F, BF16, kDensePrefix>(a, in, n, out, logits, n_cus, stream)
                : launch_network_nd<P, L, F, BF16, -1>(a, in, n, out, logits, n_cus, stream);
-}
-
-template <int P, int L, int F, bool PARTS, int ND>
-hipError_t launch_query_fp8_k(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus,
-                              hipStream_t stream)
-{
-    auto k = dev::neural_query_fp8_kernel<P, L, F, PARTS, ND>;
-    static const uint32_t bpc = blocks_per_cu(k, 64 * dev::kWavesPerBlock);
-    const uint32_t per_block = 64 * dev::kWavesPerBlock;
-    uint32_t blocks = (rb.n + per_block - 1) / per_block;
-    const uint32_t cap = a.blocks_per_cu != 0u && a.blocks_per_cu < bpc ? a.blocks_per_cu : bpc;
-    blocks = blocks < n_cus * cap ? blocks : n_cus * cap;
-    hipLaunchKernelGGL(k, dim3(blocks), dim3(per_block), 0, stream, a, rb, queue);
-    return hipGetLastError();
-}
-
-template <int P, int L, int F, int ND>
-hipError_t launch_query_fp8_nd(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus,
-                               hipStream_t stream)
-{
-    return rb.parts ? launch_query_fp8_k<P, L, F, true, ND>(a, rb, queue, n_cus, stream)
-                    : launch_query_fp8_k<P, L, F, false, ND>(a, rb, queue, n_cus, stream);
-}
-
-template <int P, int L, int F>
-hipError_t launch_query_fp8(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus, hipStream_t stream)
-{
-    return a.n_dense == (uint32_t)kDensePrefix ? launch_query_fp8_nd<P, L, F, kDensePrefix>(a, rb, queue, n_cus, stream)
-                                               : launch_query_fp8_nd<P, L, F, -1>(a, rb, queue, n_cus, stream);
 }
 
 template <int P, int L, int F, int ND>
@@ -721,11 +773,11 @@ hipError_t query_mfma(const NetArgs& a, uint32_t precision, const RayBatch& rb, 
 #define X(P_, L_, F_)                                                                 \
     if (a.n_points == P_ && a.n_levels == L_ && a.n_features == F_) {                \
         if (precision == NBVH_PREC_FP16)                                             \
-            return launch_query<P_, L_, F_, false>(a, rb, queue, n_cus, stream);          \
+            return launch_query<P_, L_, F_, NBVH_PREC_FP16>(a, rb, queue, n_cus, stream);  \
         if (precision == NBVH_PREC_BF16)                                             \
-            return launch_query<P_, L_, F_, true>(a, rb, queue, n_cus, stream);           \
+            return launch_query<P_, L_, F_, NBVH_PREC_BF16>(a, rb, queue, n_cus, stream);  \
         if (precision == NBVH_PREC_FP8 && a.mlp_frag_fp8 != nullptr)                 \
-            return launch_query_fp8<P_, L_, F_>(a, rb, queue, n_cus, stream);             \
+            return launch_query<P_, L_, F_, NBVH_PREC_FP8>(a, rb, queue, n_cus, stream);   \
     }
         NBVH_MFMA_SHAPES(X)
 #undef X

@@ -16,7 +16,6 @@ constexpr float    kInferenceMaxtEps   = 1e-3f;  // neural_bvh_renderer_constant
 constexpr float    kDepthEpsilon       = 0.2f;   // neural_bvh_module.h:270
 constexpr float    kFixedDepthEpsilon  = 1e-5f;  // neural_bvh_module.h:271
 constexpr uint32_t kDefaultMaxSteps    = 1000;   // m_max_traversal_steps, neural_bvh_module.h:200
-constexpr uint32_t kMinWaveSlots       = 4;      // fewest rays per wave a small query is spread over
 
 // One level of the multiresolution grid (tcnn GridEncoding, public convention).
 struct GridLevel {
@@ -42,6 +41,7 @@ struct NetArgs {
     uint32_t image_width;              // tiled claim order of a scanline image (0: array order)
     uint32_t queue_bands;              // ray-queue bands (1..8; 0: 8), launch shape
     uint32_t blocks_per_cu;            // persistent workgroups per CU (0: as many as fit), launch shape
+    uint32_t static_slots;             // rays per wave handed out by wave index (0: the ray queue), launcher
     const nbvh_node* nodes;            // N-BVH nodes with DILATED boxes (1 + 1e-5 about the centre)
     uint32_t n_nodes;
     uint32_t any_hit;
