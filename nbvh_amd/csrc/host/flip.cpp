@@ -4,6 +4,7 @@
 // computes the method's kernels and colour constants in FP64 (Andersson et al., HPG 2020).
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -59,38 +60,56 @@ NBVH_API int32_t nbvh_flip(nbvh_ctx* ctx, const float* d_reference, const float*
         const int rf = (int)std::ceil(3 * sd);
         if (rc > kFlipMaxRadius || rf > kFlipMaxRadius)
             fail(NBVH_ERR_UNSUPPORTED, "pixels per degree too large for the FLIP kernels' radius limit");
-        const int nc = 2 * rc + 1, nf = 2 * rf + 1;
-        // contrast sensitivity kernels: a1 sqrt(pi/b1) e^(-pi^2 d^2/b1) + a2 sqrt(pi/b2) e^(-pi^2 d^2/b2)
-        const double csf[3][4] = {{1.0, 0.0047, 0.0, 1e-5}, {1.0, 0.0053, 0.0, 1e-5}, {34.1, 0.04, 13.5, 0.025}};
-        std::vector<float> w((size_t)3 * nc * nc + 2 * (size_t)nf * nf);
-        for (int c = 0; c < 3; c++) {
-            std::vector<double> k((size_t)nc * nc);
-            double sum = 0;
-            for (int y = -rc; y <= rc; y++)
-                for (int x = -rc; x <= rc; x++) {
-                    const double d2 = ((double)x * x + (double)y * y) / (p * p);
-                    const double v = csf[c][0] * std::sqrt(kPi / csf[c][1]) * std::exp(-kPi * kPi * d2 / csf[c][1]) +
-                                     csf[c][2] * std::sqrt(kPi / csf[c][3]) * std::exp(-kPi * kPi * d2 / csf[c][3]);
-                    k[(size_t)(y + rc) * nc + (x + rc)] = v;
-                    sum += v;
-                }
-            for (size_t i = 0; i < k.size(); i++) w[(size_t)c * nc * nc + i] = (float)(k[i] / sum);
+        const int r = std::max(rc, rf);
+        std::vector<FlipTap> taps((size_t)2 * r + 1, FlipTap{});
+        // Contrast sensitivity kernels: a1 sqrt(pi/b1) e^(-pi^2 d^2/b1) + a2 sqrt(pi/b2) e^(-pi^2
+        // d^2/b2), normalised to sum 1. Each term is a product of the profiles e^(-pi^2 x^2/b)
+        // along x and y.
+        auto gauss = [&](double b, int x) { return std::exp(-kPi * kPi * ((double)x * x) / (p * p) / b); };
+        auto total = [&](double b) {
+            double s = 0;
+            for (int x = -rc; x <= rc; x++) s += gauss(b, x);
+            return s;
+        };
+        const double ab = 0.0047, rb = 0.0053, yb[2] = {0.04, 0.025}, ya[2] = {34.1, 13.5};
+        const double as = total(ab), rs = total(rb);
+        double yw[2], ysum = 0;
+        for (int k = 0; k < 2; k++) {
+            yw[k] = ya[k] * std::sqrt(kPi / yb[k]);
+            ysum += yw[k] * total(yb[k]) * total(yb[k]);
         }
-        // edge (first derivative) and point (second derivative) detectors along x, each kernel's
-        // positive and negative weights normalised to +1 and -1
-        for (int kind = 0; kind < 2; kind++) {
-            std::vector<double> k((size_t)nf * nf);
-            double pos = 0, neg = 0;
-            for (int y = -rf; y <= rf; y++)
-                for (int x = -rf; x <= rf; x++) {
-                    const double g = std::exp(-((double)x * x + (double)y * y) / (2 * sd * sd));
-                    const double v = kind == 0 ? -x * g : ((double)x * x / (sd * sd) - 1) * g;
-                    k[(size_t)(y + rf) * nf + (x + rf)] = v;
-                    if (v > 0) pos += v;
-                    if (v < 0) neg -= v;
-                }
-            float* dst = w.data() + 3 * (size_t)nc * nc + (size_t)kind * nf * nf;
-            for (size_t i = 0; i < k.size(); i++) dst[i] = (float)(k[i] > 0 ? k[i] / pos : (k[i] < 0 ? k[i] / neg : 0.0));
+        for (int x = -rc; x <= rc; x++) {
+            FlipTap& t = taps[(size_t)(x + r)];
+            t.achromatic = (float)(gauss(ab, x) / as);
+            t.red_green  = (float)(gauss(rb, x) / rs);
+            for (int k = 0; k < 2; k++) t.blue_yellow[k] = (float)gauss(yb[k], x);
+        }
+        // Edge (first derivative) and point (second derivative) detectors along x: a derivative
+        // profile times a Gaussian along y; each kernel's positive and negative weights are
+        // normalised to +1 and -1, which the sign of the x profile alone decides.
+        double gsum = 0, pos[2] = {0, 0}, neg[2] = {0, 0};
+        auto detector = [&](int kind, int x, double g) {
+            return kind == 0 ? -x * g : ((double)x * x / (sd * sd) - 1) * g;
+        };
+        for (int x = -rf; x <= rf; x++) {
+            const double g = std::exp(-((double)x * x) / (2 * sd * sd));
+            gsum += g;
+            for (int kind = 0; kind < 2; kind++) {
+                const double v = detector(kind, x, g);
+                (v > 0 ? pos : neg)[kind] += std::fabs(v);
+            }
+        }
+        for (int x = -rf; x <= rf; x++) {
+            const double g = std::exp(-((double)x * x) / (2 * sd * sd));
+            FlipTap& t = taps[(size_t)(x + r)];
+            double d[2];
+            for (int kind = 0; kind < 2; kind++) {
+                const double v = detector(kind, x, g);
+                d[kind] = v > 0 ? v / pos[kind] : (v < 0 ? v / neg[kind] : 0.0);
+            }
+            t.smooth = (float)(g / gsum);
+            t.edge   = (float)d[0];
+            t.point  = (float)d[1];
         }
         double g[3] = {0, 1, 0}, b[3] = {0, 0, 1}, lg[3], lb[3];
         hunt_lab(g, lg);
@@ -101,20 +120,19 @@ NBVH_API int32_t nbvh_flip(nbvh_ctx* ctx, const float* d_reference, const float*
         const size_t n = (size_t)width * height, tiles = flip_tiles(width, height);
         const size_t o_prep = 0, o_part = o_prep + 2 * n * 16, o_mean = o_part + tiles * 8, o_w = o_mean + 256;
         char* mem = nullptr;
-        hip_check(hipMallocAsync((void**)&mem, o_w + w.size() * 4, st), "hipMallocAsync");
+        hip_check(hipMallocAsync((void**)&mem, o_w + taps.size() * sizeof(FlipTap), st), "hipMallocAsync");
         double mean = 0;
         try {
-            hip_check(hipMemcpyAsync(mem + o_w, w.data(), w.size() * 4, hipMemcpyHostToDevice, st), "weights H2D");
+            hip_check(hipMemcpyAsync(mem + o_w, taps.data(), taps.size() * sizeof(FlipTap), hipMemcpyHostToDevice, st),
+                      "filter profiles H2D");
             FlipArgs a{};
             a.ref = d_reference;
             a.test = d_test;
             a.w = width;
             a.h = height;
-            a.rc = rc;
-            a.rf = rf;
-            a.csf = reinterpret_cast<const float*>(mem + o_w);
-            a.edge = a.csf + 3 * (size_t)nc * nc;
-            a.point = a.edge + (size_t)nf * nf;
+            a.r = r;
+            a.taps = reinterpret_cast<const FlipTap*>(mem + o_w);
+            for (int k = 0; k < 2; k++) a.by_weight[k] = (float)(yw[k] / ysum);
             a.cmax = (float)cmax;
             for (int i = 0; i < 9; i++) {
                 a.rgb2xyz[i] = (float)kRgb2Xyz[i];

@@ -158,23 +158,29 @@ struct SampleArgs {
 };
 
 // LDR-FLIP (flip.hip). Accumulation buffers are float4 per pixel (rgb sum, sample count); the
-// prepared buffers hold (Yy, Cx, Cz, Y / Yn) per pixel; kernels are (2r+1)^2 row-major with row =
-// y offset (the y feature kernels are the transposes of the x ones).
+// prepared buffers hold (Yy, Cx, Cz, Y / Yn) per pixel. A filter's profile is the same along x and
+// y; taps[t] holds all profiles at offset t - r (zero beyond a profile's own radius).
 constexpr int kFlipMaxRadius = 16;
+struct FlipTap {
+    float achromatic, red_green;  // sensitivity Gaussians, sum 1
+    float blue_yellow[2];         // the two Gaussians of the blue-yellow kernel, unnormalised
+    float smooth;                 // detector Gaussian, sum 1
+    float edge, point;            // first / second derivative, positive and negative parts sum to +-1
+    float pad;
+};
 struct FlipArgs {
-    const float* ref;   // w*h float4
-    const float* test;
-    uint32_t     w, h;
-    int          rc, rf;  // colour (contrast sensitivity) and feature kernel radii
-    const float* csf;     // 3 kernels: achromatic, red-green, blue-yellow
-    const float* edge;    // x kernel of the edge detector
-    const float* point;   // x kernel of the point detector
-    float        cmax;    // HyAB^0.7 of Hunt-adjusted green against blue
-    float        rgb2xyz[9], xyz2rgb[9], white[3], inv_white[3];
-    float*       prep_ref;   // w*h float4
-    float*       prep_test;
-    float*       map;        // optional w*h error map
-    double*      partials;   // one per 16x16 tile
+    const float*   ref;   // w*h float4
+    const float*   test;
+    uint32_t       w, h;
+    int            r;     // larger of the colour and feature radii
+    const FlipTap* taps;  // 2 r + 1
+    float          by_weight[2];  // weights of the two blue-yellow products
+    float          cmax;  // HyAB^0.7 of Hunt-adjusted green against blue
+    float          rgb2xyz[9], xyz2rgb[9], white[3], inv_white[3];
+    float*         prep_ref;   // w*h float4
+    float*         prep_test;
+    float*         map;        // optional w*h error map
+    double*        partials;   // one per tile (flip_tiles)
 };
 
 // Adam step constants (the bias correction uses each parameter's own update count).

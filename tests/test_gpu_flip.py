@@ -69,6 +69,21 @@ def test_structured_images(nb, ctx, shape):
     check_against_oracle(nb, ctx, accum(ref, 4.0), accum(np.clip(test, 0, 2), 4.0))
 
 
+@pytest.mark.parametrize("ppd,shape", [(7.0, (16, 32)), (35.0, (17, 33)), (67.02, (1, 1)), (67.02, (47, 31)),
+                                       (110.0, (50, 70)), (118.0, (5, 97))])
+def test_filter_radii_and_tile_edges(nb, ctx, ppd, shape):
+    """The separable filters from the smallest radius (1) to the largest (16), at images of one
+    pixel, exactly one 32 x 16 tile, one row and column more, and smaller than the halo. Same bars
+    as the structured images."""
+    a, b = accum(structured(*shape, 5), 4.0), accum(structured(*shape, 6), 4.0)
+    mean, m = nb.flip(ctx, a, b, ppd=ppd)
+    exp = F.flip_map(F.accum_to_linear(a), F.accum_to_linear(b), ppd)
+    d = np.abs(m.astype(np.float64) - exp)
+    assert np.quantile(d, 0.999) < 2e-2 and d.max() < 2e-2, d.max()
+    assert np.median(d) < 2e-4
+    assert abs(mean - exp.mean()) < 1e-3
+
+
 def test_neural_rendering_against_triangle_rendering(nb, ctx):
     v, t = nb.icosphere(5, seed=7, amplitude=0.1)
     scene = nb.Scene(ctx, v, t)
