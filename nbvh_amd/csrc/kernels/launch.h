@@ -22,21 +22,23 @@ inline uint32_t blocks_per_cu(K kernel, uint32_t threads)
 }
 
 // Grid of a query over rb on at most `resident` workgroups of `waves` waves, and how it hands out
-// rays. WIDE (device/grid_gather.h): at most 16 rays per wave, `step` (64 / levels) at a time.
+// rays. WIDE (device/grid_gather.h): at most wide_max rays per wave, `step` (64 / levels) at a time.
 // A batch whose rays all have a slot at once is handed out by wave index (static_slots): no queue
 // to reset before the launch, no claims, no search for work to steal at the end. Larger batches
 // and counts that live on the device take the queue, on all resident workgroups.
-// Measured for FP16 (us, whole call, queue of full waves / static LEVELS / static WIDE): 4,096 rays 267 / 160 / 90.
+// Measured (16 x 2 grid, us a call; queue of full waves / WIDE): FP16 4,096 rays 234 / 85, 16,384
+// 243 / 133, 32,384 248 / 196, 65,536 256 / 340 (32 rays per wave: full waves instead); FP32, whose
+// matrix products halve with the second segment block: 65,536 rays 618 / 471.
 struct QueryGrid {
     uint32_t blocks, static_slots;
     bool     wide;
 };
-inline QueryGrid query_grid(const RayBatch& rb, uint32_t waves, uint32_t resident, uint32_t step)
+inline QueryGrid query_grid(const RayBatch& rb, uint32_t waves, uint32_t resident, uint32_t step, uint32_t wide_max)
 {
     const uint64_t all = (uint64_t)resident * waves;
     auto blocks = [&](uint32_t slots) { return (rb.n + waves * slots - 1) / (waves * slots); };
     if (rb.live == nullptr) {
-        for (uint32_t slots = step; slots <= 16u; slots *= 2u)
+        for (uint32_t slots = step; slots <= wide_max; slots *= 2u)
             if (rb.n <= all * slots) return QueryGrid{blocks(slots), slots, true};
         if (rb.n <= all * 64u) return QueryGrid{blocks(64u), 64u, false};
     }

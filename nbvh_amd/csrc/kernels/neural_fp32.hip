@@ -51,7 +51,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void neural_query_fp32_kernel(Ne
 #pragma unroll
             for (int k = 0; k < K0; k++) x[k] = 0.f;
         }
-        // WIDE: at most 16 slots, the second block of 32 segments is empty.
+        // WIDE: at most 32 slots, the second block of 32 segments is empty.
         float z[8];
         mlp_wave_f32<K0, G == Gather::WIDE ? 1 : 2>(reinterpret_cast<const float*>(w_lds), x, z);
         if (s.state == SLOT_SEG) consume_segment<PARTS>(a, s, z, b);
@@ -106,7 +106,7 @@ static hipError_t launch_fp32_query_k(const NetArgs& a, const RayBatch& rb, uint
     auto k = dev::neural_query_fp32_kernel<P, L, F, PARTS, -1, Gather::LEVELS>;
     static const uint32_t bpc = blocks_per_cu(k, threads);
     const uint32_t cap = a.blocks_per_cu != 0u && a.blocks_per_cu < bpc ? a.blocks_per_cu : bpc;
-    const QueryGrid g = query_grid(rb, dev::kF32Waves, n_cus * cap, 64u / L < 16u ? 64u / L : 16u);
+    const QueryGrid g = query_grid(rb, dev::kF32Waves, n_cus * cap, 64u / L < 16u ? 64u / L : 16u, 32u);
     NetArgs args = a;
     args.static_slots = g.static_slots;
     if (g.static_slots == 0u) {
