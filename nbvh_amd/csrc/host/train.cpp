@@ -142,8 +142,10 @@ void trainer_step(nbvh_trainer* t, const float* d_inputs, const float* d_targets
     if (n > 0) require(d_inputs && d_targets, "NULL buffer");
     check_generation(t);
     hip_check(hipSetDevice(t->ctx->device), "hipSetDevice");
-    hip_check(train_zero(t->g_mlp.as<float>(), t->n_mlp, st), "zero");
-    hip_check(train_zero(t->loss.as<float>(), 1, st), "zero");
+    if (n == 0) {  // a batch's kernels write the whole matrix gradient and start the loss themselves
+        hip_check(train_zero(t->g_mlp.as<float>(), t->n_mlp, st), "zero");
+        hip_check(train_zero(t->loss.as<float>(), 1, st), "zero");
+    }
     bool supported = false;
     TrainArgs args = train_args(t);
     args.sample_loss = d_sample_loss;

@@ -2,19 +2,16 @@
 // replacement of the reference's trainer->training_step(stream, inputs[9 x n], targets[8 x n])
 // (src/cuda/neural/neural_bvh_renderer.cu:170-173) for its default configuration. FP32 throughout.
 //
-// Workspace: 720 activation rows of act_stride floats each (row r, sample i at r * stride + i,
-// so that a wave's 64 samples touch 256 consecutive bytes of a row), the five matrices transposed,
-// and per-chunk partial matrix gradients.
-//   train_transpose  W_l [out][in] -> W_l^T [in][out], the backward pass's row order;
-//   train_forward    one thread per sample: hash-grid features (the query's FP32 grid code) and
-//                    the MLP forward pass; each output neuron is a dot product of a weight row
-//                    (uniform across the wave, read through the scalar cache) with the lane's
-//                    activations in registers; the layer's outputs go to the activation rows
-//                    and to a per-lane LDS column from which the next layer reloads them;
-//   train_backward   one thread per sample: the composite loss of the reference's defaults
-//                    (pt_composite_loss.cuh:19-123, neural_bvh_module.h:250-266), its gradient
-//                    through the Sigmoid outputs and the ReLU layers (rows of W^T), stored per
-//                    layer, down to the feature gradients;
+// Workspace: 720 activation rows of act_stride floats each (row r, sample i at r * stride + i),
+// the weight fragments of the two passes, and per-chunk partial matrix gradients.
+//   train_fragments  the matrices as MFMA operands of the forward and the backward pass;
+//   train_forward    32 samples per wave: hash-grid features (two lanes per sample share the
+//                    levels) and the MLP on the FP32 matrix cores; every layer's outputs go to the
+//                    activation rows;
+//   train_backward   the composite loss of the reference's defaults (pt_composite_loss.cuh:19-123,
+//                    neural_bvh_module.h:250-266), its gradient through the Sigmoid outputs and the
+//                    ReLU layers (transposed fragments), stored per layer, down to the feature
+//                    gradients;
 //   train_scatter    the table gradient of levels of fewer than 128 slices of 128 KB, one
 //                    workgroup per slice: the slice is summed in LDS from every (sample, point)
 //                    whose corners fall in it and stored whole;
@@ -22,8 +19,8 @@
 //                    (count, scan, scatter), then one workgroup per slice sums its bin in LDS
 //                    and stores the slice whole; no global atomics on the gradient;
 //   train_wgrad      the matrix gradients dW[o][i] = sum over samples of delta[o] * act[i]: each
-//                    workgroup reduces one chunk of samples for one matrix through LDS tiles of 32
-//                    samples and writes its partial; train_wgrad_reduce adds the partials in
+//                    workgroup reduces one chunk of samples for one matrix on the matrix cores
+//                    through LDS tiles of 32 samples and writes its partial; train_wgrad_reduce adds the partials in
 //                    chunk order (deterministic);
 //   train_adam       tiny-cuda-nn's Adam: per-parameter update counts for the bias correction,
 //                    L2 regularisation and dense updates for the matrices, sparse updates
@@ -36,7 +33,7 @@
 #include <algorithm>
 #include <cmath>
 
-#include "../device/common.h"
+#include "../device/mlp_f32.h"
 #include "launch.h"
 
 namespace nbvh {
@@ -68,69 +65,160 @@ __device__ __forceinline__ float& row(float* act, size_t stride, int r, uint32_t
     return act[(size_t)r * stride + i];
 }
 
-// W_l^T: entry (k, o) of layer l at w_offset(l) + k * out + o.
-__global__ __launch_bounds__(256) void train_transpose_kernel(const float* __restrict__ mlp, float* __restrict__ wt)
+// MLP weight fragments of a step: the forward ones in the layout of device/mlp_f32.h
+// (F32Layout<96>), then the backward ones: matrix l transposed, rows = its inputs, k-steps over
+// its outputs. Per matrix: row block, pair of k-steps, lane, k-step of the pair, as in the forward
+// layout; inputs are ordered within a block of 32 rows like the forward rows (row 8 q + 4 g + i is
+// input 2 (16 rb + 4 q + i) + g), so that accumulators are the next product's B operands here too.
+__host__ __device__ constexpr int wt_offset(int layer)  // matrix 4 first: the order of the backward pass
+{
+    return layer == 4 ? 0 : layer == 3 ? kH * kO : kH * kO + (3 - layer) * kH * kH;
+}
+
+// Also starts the step's loss at zero.
+__global__ __launch_bounds__(256) void train_fragments_kernel(const float* __restrict__ mlp, float* __restrict__ wf,
+                                                              float* __restrict__ wb, float* __restrict__ loss)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j == 0) *loss = 0.f;
     if (j >= kMlp) return;
     const int layer = j < w_offset(1) ? 0 : j < w_offset(4) ? 1 + (j - w_offset(1)) / (kH * kH) : 4;
     const int out_w = layer == 4 ? kO : kH, in_w = layer == 0 ? kK0 : kH;
     const int local = j - w_offset(layer), o = local / in_w, k = local % in_w;
-    wt[w_offset(layer) + k * out_w + o] = mlp[j];
+    const float w = mlp[j];
+    // Row of neuron (or input) n in its block of 32, and the block.
+    auto row_of = [](int n, int& rb) {
+        const int g = n & 1, m = n >> 1;
+        rb = m / 16;
+        return 8 * ((m % 16) / 4) + 4 * g + m % 4;
+    };
+    auto at = [](int steps, int rb, int row, int kk) {
+        const int s = kk >> 1, g = kk & 1;
+        return ((rb * (steps / 2) + s / 2) * 64 + g * 32 + row) * 2 + (s & 1);
+    };
+    int rb;
+    if (layer < 4) {
+        const int row = row_of(o, rb);
+        wf[w_offset(layer) + at(in_w / 2, rb, row, k)] = w;
+    } else {
+        const int st = k >> 1, g = k & 1;
+        wf[w_offset(4) + ((st / 2 * 2 + g) * 8 + o) * 2 + (st & 1)] = w;
+    }
+    const int row = row_of(k, rb);
+    wb[wt_offset(layer) + at(out_w / 2, rb, row, o)] = w;
 }
 
-// Every lane reads back only the LDS column it wrote itself (col[k * 64 + lane]): an array with
-// run-time indices that stays out of scratch memory, with no barrier needed.
-template <int P, int L, int F>
-__global__ __launch_bounds__(64) void train_forward_kernel(TrainArgs t, const float* __restrict__ mlp,
-                                                           const float* __restrict__ in, float* __restrict__ act,
-                                                           uint32_t n)
+// A wave takes 32 samples (one MFMA block of segments): both lanes l and l + 32 work for sample
+// l, so 65,536 samples are two waves per SIMD of the whole chip. Workgroups of 8 waves (256
+// samples) share one LDS copy of the weight fragments; small batches take 2-wave workgroups so
+// that they reach every CU.
+constexpr int kWaveSamples = 32;
+constexpr uint32_t kSmallBatch = 32768;
+
+// Features of sample l on lanes l (even levels) and l + 32 (odd levels), as the B operands of layer
+// 1: x[s] holds feature 2 s on lanes 0..31 and 2 s + 1 on lanes 32..63 (one v_permlane32_swap per
+// two k-steps). The sums are those of grid_features, corner by corner.
+template <int P, int L, int F, bool EXACT>
+__device__ __forceinline__ void half_features(const NetArgs& a, const float* __restrict__ tables, const float* pts,
+                                              float* x)
 {
-    __shared__ float col[kH * 64];
-    const uint32_t lane = threadIdx.x, i = blockIdx.x * 64 + lane;
+    const uint32_t g = (threadIdx.x >> 5) & 1u;
+#pragma unroll
+    for (int l0 = 0; l0 < L; l0 += 2) {
+        const GridLevel &v0 = a.level[l0], &v1 = a.level[l0 + 1];
+        const GridLevel lv{g ? v1.scale : v0.scale, g ? v1.res : v0.res,       g ? v1.res2 : v0.res2,
+                           g ? v1.size : v0.size,   g ? v1.offset : v0.offset, g ? v1.dense : v0.dense};
+        float f[P * F];
+        if (!v0.dense && !v1.dense)  // uniform
+            gather_level_f32<P, F, true, false>(lv, tables, pts, f);
+        else
+            gather_level_f32<P, F, false, EXACT>(lv, tables, pts, f);
+#pragma unroll
+        for (int p = 0; p < P; p++)
+#pragma unroll
+            for (int k = 0; k < F; k += 2) {
+                const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(f[p * F + k]),
+                                                                __float_as_uint(f[p * F + k + 1]), false, false);
+                x[(p * L + l0) * (F / 2) + k / 2]     = __uint_as_float(r[0]);
+                x[(p * L + l0 + 1) * (F / 2) + k / 2] = __uint_as_float(r[1]);
+            }
+    }
+}
+
+// acc[rb] += (RB blocks of 32 rows of the S k-steps' weights) x b[s].
+template <int S, int RB>
+__device__ __forceinline__ void train_layer(const float* w, const float* b, floatx16_t* acc)
+{
+    const float2* w2 = reinterpret_cast<const float2*>(w) + (threadIdx.x & 63u);
+#pragma unroll
+    for (int s = 0; s < S; s += 2) {
+        float2 v[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; rb++) v[rb] = w2[(rb * (S / 2) + s / 2) * 64];
+#pragma unroll
+        for (int e = 0; e < 2; e++)
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++)
+                acc[rb] = __builtin_amdgcn_mfma_f32_32x32x2f32(e ? v[rb].y : v[rb].x, b[s + e], acc[rb], 0, 0, 0);
+    }
+}
+
+// The forward pass on the FP32 matrix cores (bit-identical to fmaf chains with k ascending, see
+// device/mlp_f32.h). Per layer the 64 activations of a sample sit in two lanes, k = 2 s + l / 32 in
+// register s, which are stored to the activation rows (128 B per half wave) and feed the next layer.
+// Measured per 65,536 samples of the 16 x 2 grid: 167 us, against 258 us with one thread per
+// sample and weights through the scalar cache; what is left is the gathers and 92 MB of rows.
+template <int P, int L, int F, int W>
+__global__ __launch_bounds__(64 * W, 2) void train_forward_kernel(TrainArgs t, const float* __restrict__ wf,
+                                                                 const float* __restrict__ in,
+                                                                 float* __restrict__ act, uint32_t n)
+{
+    __shared__ float4 w_lds[kMlp / 4];
+    for (uint32_t j = threadIdx.x; j < (uint32_t)kMlp / 4u; j += 64u * W)
+        w_lds[j] = reinterpret_cast<const float4*>(wf)[j];
+    const uint32_t lane = threadIdx.x & 63u, g = lane >> 5;
+    const uint32_t i = (blockIdx.x * W + (threadIdx.x >> 6)) * kWaveSamples + (lane & 31u);
     const size_t S = t.act_stride;
-    float pts[3 * P];
     const bool ok = i < n;
+    float pts[3 * P], x[kK0 / 2];
 #pragma unroll
     for (int c = 0; c < 3 * P; c++) pts[c] = ok ? in[(size_t)i * (3 * P) + c] : 0.5f;
-    float x[kK0];
-    grid_features<P, L, F, float>(t.net, t.tables, pts, x);  // wave-uniform, every lane takes part
-    if (!ok) return;
+    if (__all(in_unit_cube<3 * P>(pts)))
+        half_features<P, L, F, false>(t.net, t.tables, pts, x);
+    else
+        half_features<P, L, F, true>(t.net, t.tables, pts, x);
+    __syncthreads();
+    const float* w = reinterpret_cast<const float*>(w_lds);
+    if (ok) {
 #pragma unroll
-    for (int k = 0; k < kK0; k++) row(act, S, kA0 + k, i) = x[k];
-    for (int o = 0; o < kH; o++) {
-        const float* w = mlp + o * kK0;
-        float s = 0.f;
-#pragma unroll
-        for (int k = 0; k < kK0; k++) s = fmaf(w[k], x[k], s);
-        s = fmaxf(s, 0.f);
-        col[o * 64 + lane] = s;
-        row(act, S, kHid + o, i) = s;
+        for (int s = 0; s < kK0 / 2; s++) row(act, S, kA0 + 2 * s + g, i) = x[s];
     }
-    float h[kH];
-    for (int layer = 1; layer < 4; layer++) {
+    floatx16_t acc[2] = {};
+    train_layer<kK0 / 2, 2>(w, x, acc);
+    float b[kH / 2];
 #pragma unroll
-        for (int k = 0; k < kH; k++) h[k] = col[k * 64 + lane];
-        const float* W = mlp + w_offset(layer);
-        for (int o = 0; o < kH; o++) {
-            const float* w = W + o * kH;
-            float s = 0.f;
+    for (int layer = 0; layer < 4; layer++) {
 #pragma unroll
-            for (int k = 0; k < kH; k++) s = fmaf(w[k], h[k], s);
-            s = fmaxf(s, 0.f);
-            col[o * 64 + lane] = s;
-            row(act, S, kHid + layer * kH + o, i) = s;
+        for (int s = 0; s < kH / 2; s++) b[s] = fmaxf(acc[s / 16][s % 16], 0.f);
+        if (ok) {
+#pragma unroll
+            for (int s = 0; s < kH / 2; s++) row(act, S, kHid + layer * kH + 2 * s + g, i) = b[s];
         }
+        if (layer == 3) break;
+        acc[0] = acc[1] = floatx16_t{};
+        train_layer<kH / 2, 2>(w + w_offset(layer + 1), b, acc);
     }
+    floatx16_t out = {};
+    const float2* wo = reinterpret_cast<const float2*>(w + w_offset(4));
 #pragma unroll
-    for (int k = 0; k < kH; k++) h[k] = col[k * 64 + lane];
-    const float* W = mlp + w_offset(4);
+    for (int s = 0; s < kH / 2; s += 2) {
+        const float2 v = wo[(s + g) * 8 + (lane & 7u)];
+        out = __builtin_amdgcn_mfma_f32_32x32x2f32(v.x, b[s], out, 0, 0, 0);
+        out = __builtin_amdgcn_mfma_f32_32x32x2f32(v.y, b[s + 1], out, 0, 0, 0);
+    }
+    if (ok) {
 #pragma unroll
-    for (int o = 0; o < kO; o++) {
-        float s = 0.f;
-#pragma unroll
-        for (int k = 0; k < kH; k++) s = fmaf(W[o * kH + k], h[k], s);
-        row(act, S, kY + o, i) = sigmoidf_cw(s);
+        for (int r = 0; r < 4; r++) row(act, S, kY + 4 * g + r, i) = sigmoidf_cw(out[r]);
     }
 }
 
@@ -162,71 +250,74 @@ __device__ __forceinline__ void element_loss(int j, float y, float target, bool 
     }
 }
 
-template <int P, int L, int F>
-__global__ __launch_bounds__(64) void train_backward_kernel(TrainArgs t, const float* __restrict__ wt,
-                                                            const float* __restrict__ in,
-                                                            const float* __restrict__ targets,
-                                                            float* __restrict__ act, uint32_t n)
+// The backward pass, 32 samples per wave like the forward pass: delta of layer l - 1 = W_l^T delta_l
+// where the activation is positive, with the outputs o ascending (the transposed fragments).
+// Measured per 65,536 samples: 102 us (154 us with one thread per sample); 260 MB of rows.
+template <int W>
+__global__ __launch_bounds__(64 * W, 2) void train_backward_kernel(TrainArgs t, const float* __restrict__ wb,
+                                                                  const float* __restrict__ targets,
+                                                                  float* __restrict__ act, uint32_t n)
 {
-    __shared__ float col[kH * 64];
-    const uint32_t lane = threadIdx.x, i = blockIdx.x * 64 + lane;
+    __shared__ float4 w_lds[kMlp / 4];
+    for (uint32_t j = threadIdx.x; j < (uint32_t)kMlp / 4u; j += 64u * W)
+        w_lds[j] = reinterpret_cast<const float4*>(wb)[j];
+    const uint32_t lane = threadIdx.x & 63u, g = lane >> 5;
+    const uint32_t i = (blockIdx.x * W + (threadIdx.x >> 6)) * kWaveSamples + (lane & 31u);
     const size_t S = t.act_stride;
     const bool ok = i < n;
     const float inv_n = 1.f / ((float)n * (float)kO);
+    // Both lanes of a sample form its 8 output deltas; lane l + 32 keeps the odd ones.
     float dz[kO], lsum = 0.f;
+#pragma unroll
+    for (int j = 0; j < kO; j++) dz[j] = 0.f;
     if (ok) {
         const bool keep = targets[(size_t)i * kO] >= 0.5f;
 #pragma unroll
         for (int j = 0; j < kO; j++) {
             const float y = row(act, S, kY + j, i);
-            float l, g;
-            element_loss(j, y, targets[(size_t)i * kO + j], keep, l, g);
+            float l, gr;
+            element_loss(j, y, targets[(size_t)i * kO + j], keep, l, gr);
             lsum += l * inv_n;
-            dz[j] = (g * inv_n) * (y * (1.f - y));  // through the Sigmoid output activation
-            row(act, S, kD5 + j, i) = dz[j];
+            dz[j] = (gr * inv_n) * (y * (1.f - y));  // through the Sigmoid output activation
         }
-        if (t.sample_loss) t.sample_loss[i] = lsum;  // this sample's element values, in element order
+        if (t.sample_loss && g == 0u) t.sample_loss[i] = lsum;  // the element values in element order
     }
+    float b[kH / 2];
+#pragma unroll
+    for (int s = 0; s < kO / 2; s++) b[s] = g ? dz[2 * s + 1] : dz[2 * s];
+    if (ok) {
+#pragma unroll
+        for (int s = 0; s < kO / 2; s++) row(act, S, kD5 + 2 * s + g, i) = b[s];
+    }
+    if (g != 0u) lsum = 0.f;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
     if (lane == 0) atomicAdd(t.loss, lsum);
-    if (!ok) return;
-    // delta of h4 from the output matrix (rows of W4^T), then down the ReLU layers.
-    {
-        const float* T = wt + w_offset(4);
-        for (int k = 0; k < kH; k++) {
-            float s = 0.f;
+    __syncthreads();
+    const float* w = reinterpret_cast<const float*>(w_lds);
 #pragma unroll
-            for (int o = 0; o < kO; o++) s = fmaf(T[k * kO + o], dz[o], s);
-            s = row(act, S, kHid + 3 * kH + k, i) > 0.f ? s : 0.f;
-            col[k * 64 + lane] = s;
-            row(act, S, kD + 3 * kH + k, i) = s;
+    for (int layer = 3; layer >= 0; layer--) {  // delta of h(layer + 1)
+        float h[kH / 2];
+#pragma unroll
+        for (int s = 0; s < kH / 2; s++) h[s] = ok ? row(act, S, kHid + layer * kH + 2 * s + g, i) : 0.f;
+        floatx16_t acc[2] = {};
+        if (layer == 3)
+            train_layer<kO / 2, 2>(w + wt_offset(4), b, acc);
+        else
+            train_layer<kH / 2, 2>(w + wt_offset(layer + 1), b, acc);
+#pragma unroll
+        for (int s = 0; s < kH / 2; s++) b[s] = h[s] > 0.f ? acc[s / 16][s % 16] : 0.f;
+        if (ok) {
+#pragma unroll
+            for (int s = 0; s < kH / 2; s++) row(act, S, kD + layer * kH + 2 * s + g, i) = b[s];
         }
     }
-    float d[kH];
-    for (int layer = 3; layer >= 1; layer--) {
+    // Feature gradients; train_scatter adds them into the tables' gradient.
+    floatx16_t acc[3] = {};
+    train_layer<kH / 2, 3>(w + wt_offset(0), b, acc);
+    if (ok) {
 #pragma unroll
-        for (int k = 0; k < kH; k++) d[k] = col[k * 64 + lane];
-        const float* T = wt + w_offset(layer);
-        for (int k = 0; k < kH; k++) {
-            float s = 0.f;
-#pragma unroll
-            for (int o = 0; o < kH; o++) s = fmaf(T[k * kH + o], d[o], s);
-            s = row(act, S, kHid + (layer - 1) * kH + k, i) > 0.f ? s : 0.f;
-            col[k * 64 + lane] = s;
-            row(act, S, kD + (layer - 1) * kH + k, i) = s;
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < kH; k++) d[k] = col[k * 64 + lane];  // delta of h1
-    // Feature gradients (rows of W0^T); train_scatter adds them into the tables' gradient.
-#pragma unroll 4
-    for (int k = 0; k < kK0; k++) {
-        const float* T = wt + k * kH;
-        float s = 0.f;
-#pragma unroll
-        for (int o = 0; o < kH; o++) s = fmaf(T[o], d[o], s);
-        row(act, S, kDX + k, i) = s;
+        for (int s = 0; s < kK0 / 2; s++) row(act, S, kDX + 2 * s + g, i) = acc[s / 16][s % 16];
     }
 }
 
@@ -552,47 +643,74 @@ __global__ __launch_bounds__(kScatterThreads) void train_bin_accumulate_kernel(T
     for (uint32_t j = threadIdx.x; j < len * F / 4; j += kScatterThreads) out[j] = acc4[j];
 }
 
-// Partial dW[o][k] = sum over samples b in [b0, b1) of delta_b[o] * act_b[k] for one matrix
-// (O outputs, I inputs): tiles of 32 samples of the O delta rows and the I activation rows are
-// staged in LDS (sm, (O + I) x 33 floats), each thread accumulates an MO x MK block.
+// Partial dW[o][k] = sum over samples b in [b0, b1) of delta_b[o] * act_b[k] for one matrix (O
+// outputs, I inputs), b ascending: tiles of 32 samples of the O delta rows and the I activation rows
+// are staged in LDS (sm, (O + I) x 33 floats); the 32 x 32 blocks of the matrix go round the
+// workgroup's 4 waves, each block a chain of v_mfma_f32_32x32x2_f32 over the samples.
+// Measured per 65,536 samples (all five matrices): 44 us; 92 us with FMAs on LDS operands, and 91
+// on the matrix cores without the next tile's loads in flight.
 template <int O, int I>
 __device__ __forceinline__ void wgrad_chunk(const float* __restrict__ act, size_t S, int d_row, int a_row, uint32_t b0,
                                             uint32_t b1, float* sm, float* __restrict__ out)
 {
-    constexpr int TO = O < 16 ? O : 16, TK = 256 / TO, MO = O / TO, MK = I / TK;
-    static_assert(TO * MO == O && TK * MK == I, "tile shape");
-    const int tid = threadIdx.x, og = tid / TK, kg = tid % TK;
-    float acc[MO][MK];
+    constexpr int RB = (O + 31) / 32, CB = I / 32, BLOCKS = RB * CB, PER = (BLOCKS + 3) / 4;
+    static_assert(I % 32 == 0 && (O % 32 == 0 || O < 32), "blocks of 32 x 32");
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, c = lane & 31;
+    floatx16_t acc[PER] = {};
+    // Four samples of a row per load (rows and chunks start at multiples of 32 samples; a row has
+    // at least the samples up to the next multiple of 32); the next tile is loaded while this
+    // one is multiplied.
+    constexpr int QUADS = (O + I) * 8, LOADS = (QUADS + 255) / 256;
+    float4 v[LOADS];
+    auto load = [&](uint32_t c0) {
 #pragma unroll
-    for (int m = 0; m < MO; m++)
-#pragma unroll
-        for (int q = 0; q < MK; q++) acc[m][q] = 0.f;
+        for (int m = 0; m < LOADS; m++) {
+            const int e = tid + m * 256, r = e >> 3;
+            const int src = r < O ? d_row + r : a_row + (r - O);
+            if (e < QUADS) v[m] = *reinterpret_cast<const float4*>(act + (size_t)src * S + c0 + 4 * (e & 7));
+        }
+    };
+    if (b0 < b1) load(b0);
     for (uint32_t c0 = b0; c0 < b1; c0 += 32) {
         __syncthreads();
-        for (int e = tid; e < (O + I) * 32; e += 256) {
-            const int r = e >> 5, j = e & 31;
-            const uint32_t b = c0 + j;
-            const int src = r < O ? d_row + r : a_row + (r - O);
-            sm[r * 33 + j] = b < b1 ? act[(size_t)src * S + b] : 0.f;
+#pragma unroll
+        for (int m = 0; m < LOADS; m++) {
+            const int e = tid + m * 256;
+            if (e < QUADS) {
+                const uint32_t b = c0 + 4 * (e & 7);
+                float* d = sm + (e >> 3) * 33 + 4 * (e & 7);
+                d[0] = b < b1 ? v[m].x : 0.f;
+                d[1] = b + 1 < b1 ? v[m].y : 0.f;
+                d[2] = b + 2 < b1 ? v[m].z : 0.f;
+                d[3] = b + 3 < b1 ? v[m].w : 0.f;
+            }
         }
         __syncthreads();
-#pragma unroll 4
-        for (int j = 0; j < 32; j++) {
-            float dv[MO], av[MK];
+        if (c0 + 32 < b1) load(c0 + 32);
 #pragma unroll
-            for (int m = 0; m < MO; m++) dv[m] = sm[(og * MO + m) * 33 + j];
+        for (int q = 0; q < PER; q++) {
+            const int blk = wave + 4 * q;
+            if (blk < BLOCKS) {
+                // Rows past O (the 8-output matrix) repeat its rows; their products are not stored.
+                const float* d = sm + ((blk / CB) * 32 + c) % O * 33 + g;
+                const float* x = sm + (O + (blk % CB) * 32 + c) * 33 + g;
 #pragma unroll
-            for (int q = 0; q < MK; q++) av[q] = sm[(O + kg * MK + q) * 33 + j];
-#pragma unroll
-            for (int m = 0; m < MO; m++)
-#pragma unroll
-                for (int q = 0; q < MK; q++) acc[m][q] = fmaf(dv[m], av[q], acc[m][q]);
+                for (int s = 0; s < 16; s++)
+                    acc[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(d[2 * s], x[2 * s], acc[q], 0, 0, 0);
+            }
         }
     }
 #pragma unroll
-    for (int m = 0; m < MO; m++)
+    for (int q = 0; q < PER; q++) {
+        const int blk = wave + 4 * q;
+        if (blk < BLOCKS) {
 #pragma unroll
-        for (int q = 0; q < MK; q++) out[(og * MO + m) * I + kg * MK + q] = acc[m][q];
+            for (int r = 0; r < 16; r++) {
+                const int o = (blk / CB) * 32 + 8 * (r / 4) + 4 * g + r % 4;
+                if (o < O) out[o * I + (blk % CB) * 32 + c] = acc[q][r];
+            }
+        }
+    }
 }
 
 // Workgroup (chunk c, matrix l): the partial of samples [c * per, min(n, (c + 1) * per)).
@@ -668,7 +786,7 @@ uint32_t train_act_stride(uint32_t max_batch) { return (max_batch + 63u) & ~63u;
 
 size_t train_act_bytes(uint32_t max_batch)
 {
-    return ((size_t)dev::kRows * train_act_stride(max_batch) + (size_t)dev::kMlp * (1 + dev::kChunks)) * sizeof(float);
+    return ((size_t)dev::kRows * train_act_stride(max_batch) + (size_t)dev::kMlp * (2 + dev::kChunks)) * sizeof(float);
 }
 
 hipError_t train_zero(float* p, uint64_t n, hipStream_t stream)
@@ -698,9 +816,13 @@ hipError_t train_gradients(const TrainArgs& t, const float* in, const float* tar
     const NetArgs& a   = t.net;
     const size_t   S   = t.act_stride;
     float* const   act = t.act;
-    float* const   wt  = act + (size_t)dev::kRows * S;
-    float* const   part = wt + dev::kMlp;
-    const dim3 grid((n + 63) / 64), block(64), grid_mlp((dev::kMlp + 255) / 256);
+    float* const   wf  = act + (size_t)dev::kRows * S;  // rows of a multiple of 64 floats: 16-byte aligned
+    float* const   wb  = wf + dev::kMlp;
+    float* const   part = wb + dev::kMlp;
+    const dim3 grid_mlp((dev::kMlp + 255) / 256);
+    const bool small = n <= dev::kSmallBatch;
+    const uint32_t per_wg = (small ? 2u : 8u) * dev::kWaveSamples;
+    const dim3 grid((n + per_wg - 1) / per_wg), block((small ? 2u : 8u) * 64u);
     if (a.n_levels > (uint32_t)kMaxLevels || a.n_features == 0) return hipErrorInvalidValue;
     // Levels of at least NBVH_BIN_MIN_SLICES slices (16 MB of gradient) take the binned path; the
     // others are scanned once per slice, split into parts so that each workgroup adds about 32K
@@ -745,14 +867,20 @@ hipError_t train_gradients(const TrainArgs& t, const float* in, const float* tar
     uint32_t* const term_r  = cursors + (kMaxBins + 1);
     float* const    term_v  = reinterpret_cast<float*>(term_r + (size_t)S * a.n_points * a.n_levels * 8u);
     const dim3 bin_grid((n * a.n_points + dev::kBinPairs - 1) / dev::kBinPairs, bins.count, windows);
-    // Split slices add into the gradient with global atomics: their levels start from zero. Every
-    // other entry is stored by its slice.
-    for (uint32_t l = 0; l < a.n_levels; l++)
-        if (map.parts[l] > 1) {
-            const hipError_t e = train_zero(t.grad_tables + (size_t)a.level[l].offset * a.n_features,
-                                            (uint64_t)a.level[l].size * a.n_features, stream);
-            if (e != hipSuccess) return e;
+    // Split slices add into the gradient with global atomics: their levels start from zero, one
+    // launch for each run of them. Every other entry is stored by its slice.
+    for (uint32_t l = 0; l < a.n_levels;) {
+        if (map.parts[l] <= 1) {
+            l++;
+            continue;
         }
+        const uint32_t first = a.level[l].offset;
+        uint64_t end = first;
+        for (; l < a.n_levels && map.parts[l] > 1; l++) end = (uint64_t)a.level[l].offset + a.level[l].size;
+        const hipError_t e =
+            train_zero(t.grad_tables + (size_t)first * a.n_features, (end - first) * a.n_features, stream);
+        if (e != hipSuccess) return e;
+    }
     if (n_bins > 0) {
         const hipError_t e = train_zero(reinterpret_cast<float*>(counts), n_bins, stream);
         if (e != hipSuccess) return e;
@@ -761,10 +889,19 @@ hipError_t train_gradients(const TrainArgs& t, const float* in, const float* tar
 #define X(P_, L_, F_)                                                                                                \
     if (a.n_points == P_ && a.n_levels == L_ && a.n_features == F_) {                                                \
         shape = true;                                                                                                \
-        hipLaunchKernelGGL(dev::train_transpose_kernel, grid_mlp, dim3(256), 0, stream, t.mlp, wt);                  \
-        hipLaunchKernelGGL((dev::train_forward_kernel<P_, L_, F_>), grid, block, 0, stream, t, t.mlp, in, act, n);    \
-        hipLaunchKernelGGL((dev::train_backward_kernel<P_, L_, F_>), grid, block, 0, stream, t, (const float*)wt, in, \
-                           targets, act, n);                                                                         \
+        hipLaunchKernelGGL(dev::train_fragments_kernel, grid_mlp, dim3(256), 0, stream, t.mlp, wf, wb, t.loss);      \
+        if (small)                                                                                                   \
+            hipLaunchKernelGGL((dev::train_forward_kernel<P_, L_, F_, 2>), grid, block, 0, stream, t,                \
+                               (const float*)wf, in, act, n);                                                        \
+        else                                                                                                         \
+            hipLaunchKernelGGL((dev::train_forward_kernel<P_, L_, F_, 8>), grid, block, 0, stream, t,                \
+                               (const float*)wf, in, act, n);                                                        \
+        if (small)                                                                                                   \
+            hipLaunchKernelGGL(dev::train_backward_kernel<2>, grid, block, 0, stream, t, (const float*)wb, targets,  \
+                               act, n);                                                                              \
+        else                                                                                                         \
+            hipLaunchKernelGGL(dev::train_backward_kernel<8>, grid, block, 0, stream, t, (const float*)wb, targets,  \
+                               act, n);                                                                              \
         if (map.first[L_] > 0)                                                                                       \
             hipLaunchKernelGGL((dev::train_scatter_kernel<P_, L_, F_>), dim3(map.first[L_]), dim3(dev::kScatterThreads), \
                                0, stream, t, map, in, (const float*)act, t.grad_tables, n);                          \

@@ -75,6 +75,28 @@ def test_gradients_match_oracle(nb, orc, ctx, setup, n):
                      setup["x"][:n], setup["t"][:n])
 
 
+@pytest.mark.parametrize("n", [1, 31, 33, 63, 65, 257, 32769])
+def test_gradients_at_wave_and_workgroup_edges(nb, orc, ctx, setup, n):
+    """The matrix-core passes take 32 samples per wave, in workgroups of 64 samples up to 32,768
+    samples and of 256 beyond; the matrix gradients take tiles of 32 samples, four per load. One
+    sample, one less and one more than each, and the first batch of the large workgroups (the
+    setup's segments repeated). Same bars as the other batches; the smallest ones touch too few
+    entries for the count that _check_gradients asks for and are compared here."""
+    from oracle import train
+    reps = -(-n // len(setup["x"]))
+    x, t = np.tile(setup["x"], (reps, 1))[:n], np.tile(setup["t"], (reps, 1))[:n]
+    tr = nb.Trainer(ctx, setup["scene"], max_batch=n)
+    loss = tr.step(x, t, gradients_only=True)
+    gt, gm = tr.get(nb.TRAIN_GRAD_TABLES), tr.get(nb.TRAIN_GRAD_MLP)
+    l64, dt64, dm64, _ = train.train_gradients(setup["net"].levels(), setup["cfg"], setup["tables"].astype(np.float64),
+                                               setup["mlp"].astype(np.float64), x.astype(np.float64),
+                                               t.astype(np.float64))
+    assert abs(loss - l64) <= 1e-4 * abs(l64)
+    assert np.linalg.norm(gm - dm64) <= 1e-4 * np.linalg.norm(dm64)
+    assert np.linalg.norm(gt - dt64) <= 1e-3 * np.linalg.norm(dt64)
+    tr.close()
+
+
 @pytest.mark.parametrize("n", [1, 2000])
 def test_chess_shape_gradients_match_oracle(nb, orc, ctx, setup, n):
     """The (3, 8, 4) shape of the reference's chess configuration (8 levels x 4 features, 2^18
