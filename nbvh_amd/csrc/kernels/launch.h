@@ -24,8 +24,9 @@ inline uint32_t blocks_per_cu(K kernel, uint32_t threads)
 // Grid of a query over rb on at most `resident` workgroups of `waves` waves, and how it hands out
 // rays. WIDE (device/grid_gather.h): at most wide_max rays per wave, `step` (64 / levels) at a time.
 // A batch whose rays all have a slot at once is handed out by wave index (static_slots): no queue
-// to reset before the launch, no claims, no search for work to steal at the end. Larger batches
-// and counts that live on the device take the queue, on all resident workgroups.
+// to reset before the launch, no claims, no search for work to steal at the end. rb.n is what
+// counts: with a count on the device (at most n) the waves past it end at once. Larger batches
+// take the queue, on all resident workgroups.
 // Measured (16 x 2 grid, us a call; queue of full waves / WIDE): FP16 4,096 rays 234 / 85, 16,384
 // 243 / 133, 32,384 248 / 196, 65,536 256 / 340 (32 rays per wave: full waves instead); FP32, whose
 // matrix products halve with the second segment block: 65,536 rays 618 / 471.
@@ -37,11 +38,9 @@ inline QueryGrid query_grid(const RayBatch& rb, uint32_t waves, uint32_t residen
 {
     const uint64_t all = (uint64_t)resident * waves;
     auto blocks = [&](uint32_t slots) { return (rb.n + waves * slots - 1) / (waves * slots); };
-    if (rb.live == nullptr) {
-        for (uint32_t slots = step; slots <= wide_max; slots *= 2u)
-            if (rb.n <= all * slots) return QueryGrid{blocks(slots), slots, true};
-        if (rb.n <= all * 64u) return QueryGrid{blocks(64u), 64u, false};
-    }
+    for (uint32_t slots = step; slots <= wide_max; slots *= 2u)
+        if (rb.n <= all * slots) return QueryGrid{blocks(slots), slots, true};
+    if (rb.n <= all * 64u) return QueryGrid{blocks(64u), 64u, false};
     return QueryGrid{resident, 0u, false};
 }
 
