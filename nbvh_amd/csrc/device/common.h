@@ -343,90 +343,6 @@ __device__ __forceinline__ float half_bits_to_float(uint32_t bits16)
     return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16);
 }
 
-// Trilinear interpolation of the F features of one level at point (x, y, z):
-// acc[f] = sum over corners c = 0..7 of fmaf(w_c, v_c[f], .), tcnn's corner order.
-// Tables: FP32 (T = float) or IEEE half bits (T = uint16_t), entries of F consecutive values.
-template <int F, typename T, bool EXACT>
-__device__ __forceinline__ void interp_level(const GridLevel& L, const T* __restrict__ table, float x, float y, float z,
-                                             float acc[F])
-{
-    uint32_t g[3];
-    float f[3];
-    grid_cell(L, x, y, z, g, f);
-    uint32_t idx[8];
-    grid_corners<EXACT>(L, g, idx);
-    const T* base = table + (size_t)L.offset * F;
-#pragma unroll
-    for (int k = 0; k < F; k++) acc[k] = 0.f;
-#pragma unroll
-    for (uint32_t c = 0; c < 8; c++) {
-        const float w = corner_weight(c, f);
-        const T* v = base + (size_t)idx[c] * F;
-        float val[F];
-        if constexpr (sizeof(T) == 4) {
-            if constexpr (F == 2) {
-                const float2 q = *reinterpret_cast<const float2*>(v);
-                val[0] = q.x;
-                val[1] = q.y;
-            } else if constexpr (F == 4) {
-                const float4 q = *reinterpret_cast<const float4*>(v);
-                val[0] = q.x;
-                val[1] = q.y;
-                val[2] = q.z;
-                val[3] = q.w;
-            } else {
-#pragma unroll
-                for (int k = 0; k < F; k++) val[k] = (float)v[k];
-            }
-        } else {
-            if constexpr (F == 2) {
-                const uint32_t q = *reinterpret_cast<const uint32_t*>(v);
-                val[0] = half_bits_to_float(q & 0xFFFFu);
-                val[1] = half_bits_to_float(q >> 16);
-            } else if constexpr (F == 4) {
-                const uint2 q = *reinterpret_cast<const uint2*>(v);
-                val[0] = half_bits_to_float(q.x & 0xFFFFu);
-                val[1] = half_bits_to_float(q.x >> 16);
-                val[2] = half_bits_to_float(q.y & 0xFFFFu);
-                val[3] = half_bits_to_float(q.y >> 16);
-            } else {
-#pragma unroll
-                for (int k = 0; k < F; k++) val[k] = half_bits_to_float(v[k]);
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < F; k++) acc[k] = fmaf(w, val[k], acc[k]);
-    }
-}
-
-// Hash-grid features of P points: x[p*L*F + l*F + f].
-template <int P, int L, int F, typename T, bool EXACT>
-__device__ __forceinline__ void grid_features_impl(const NetArgs& a, const T* __restrict__ table, const float* pts,
-                                                   float* x)
-{
-#pragma unroll
-    for (int p = 0; p < P; p++) {
-#pragma unroll
-        for (int l = 0; l < L; l++) {
-            float acc[F];
-            interp_level<F, T, EXACT>(a.level[l], table, pts[3 * p], pts[3 * p + 1], pts[3 * p + 2], acc);
-#pragma unroll
-            for (int k = 0; k < F; k++) x[p * L * F + l * F + k] = acc[k];
-        }
-    }
-}
-
-// One wave-uniform decision per call: the branch-free indexing when every lane's points are in
-// the unit cube (the normal case: segments inside the neural scene box), else the exact modulo.
-template <int P, int L, int F, typename T>
-__device__ __forceinline__ void grid_features(const NetArgs& a, const T* __restrict__ table, const float* pts, float* x)
-{
-    if (__all(in_unit_cube<3 * P>(pts)))
-        grid_features_impl<P, L, F, T, false>(a, table, pts, x);
-    else
-        grid_features_impl<P, L, F, T, true>(a, table, pts, x);
-}
-
 // LocalT depth decode (include/cuda/neural/neural_bvh_module_common.cuh:32-57); FLT_MAX = rejected.
 // The reference evaluates (segment_length + 1e-3) in double (double literal); FP32 here.
 __device__ __forceinline__ float decode_depth(float u, float mint, float maxt)

@@ -37,10 +37,11 @@ __device__ __forceinline__ float trilinear_weight(int c, const float wx[2], cons
 
 // How a wave gathers the features of its slots.
 //   LEVELS  every lane its own segment, level after level (the three points of a level together);
-//   PHASES  the same, the hashed levels in the order of level_phases;
+//   PAIRS   the same two levels at a time: twice the loads in flight, for launches with few waves;
+//   PHASES  level by level, the hashed levels in the order of level_phases;
 //   WIDE    few slots per wave: a lane takes one level of one slot, 64 / L slots at a time, so that
 //           a segment costs one memory round trip instead of one per level.
-enum class Gather { LEVELS, PHASES, WIDE };
+enum class Gather { LEVELS, PHASES, WIDE, PAIRS };
 
 // Visit each of N levels once, f(level) with a wave-uniform level, starting with the level whose
 // turn it is: the turn moves every kLevelTicks of the 100 MHz clock, alike on every CU. The tables

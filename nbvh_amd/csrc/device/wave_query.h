@@ -248,7 +248,12 @@ __device__ __forceinline__ uint32_t first_rays(const NetArgs& a, const RayBatch&
 {
     const uint32_t lane = threadIdx.x & 63u, per_block = blockDim.x >> 6, waves = gridDim.x * per_block;
     if (a.static_slots != 0u) {
-        const uint32_t i = (blockIdx.x * per_block + (threadIdx.x >> 6)) * a.static_slots + lane;
+        // A count on the device may fill only part of the launch: its rays go to the first wave of
+        // every workgroup, then to the second, so that they reach all CUs; a full launch keeps
+        // neighbouring rays in a workgroup.
+        const uint32_t w = threadIdx.x >> 6;
+        const uint32_t wave = b.live ? w * gridDim.x + blockIdx.x : blockIdx.x * per_block + w;
+        const uint32_t i = wave * a.static_slots + lane;
         s.state = SLOT_DONE;
         if (lane < a.static_slots && i < q.n_rays) {
             s.state = SLOT_NEW;

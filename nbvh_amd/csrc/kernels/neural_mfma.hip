@@ -105,29 +105,33 @@ __device__ __forceinline__ void level_offsets(const GridLevel& lv, float x, floa
     for (int c = 0; c < 8; c++) off[c] = (idx[c] + lv.offset) << kShift;
 }
 
-// One level, all P points: the 8 P corner offsets, then all loads, then the corner weights and the
-// FP32 accumulation over corners 0..7 (tcnn's trilinear weights). out[p * F / 2 ..]: the level's
-// features of point p as 16-bit pairs.
-template <int P, int F, bool BF16, bool HASHED, bool EXACT>
-__device__ __forceinline__ void gather_level(const GridLevel& lv, __amdgpu_buffer_rsrc_t tab, const float* pts,
+// NL consecutive levels (lv[0 .. NL)), all P points: the corner offsets, then all 8 NL P loads, then
+// the corner weights and the FP32 accumulation over corners 0..7 (tcnn's trilinear weights).
+// out[(l * P + p) * F / 2 ..]: the features of point p at level l as 16-bit pairs.
+template <int P, int F, bool BF16, bool HASHED, bool EXACT, int NL = 1>
+__device__ __forceinline__ void gather_level(const GridLevel* lv, __amdgpu_buffer_rsrc_t tab, const float* points,
                                              uint32_t* out)
 {
+    constexpr int N = NL * P;
     typedef typename Frag<BF16>::elem E;
     typedef E pair_t __attribute__((ext_vector_type(2)));
-    uint32_t off[P][8];
-    float fr[P][3];
+    uint32_t off[N][8];
+    float fr[N][3];
 #pragma unroll
-    for (int p = 0; p < P; p++)
-        level_offsets<F, HASHED, EXACT>(lv, pts[3 * p], pts[3 * p + 1], pts[3 * p + 2], off[p], fr[p]);
+    for (int p = 0; p < N; p++)
+    {
+        const float* pt = points + 3 * (p % P);
+        level_offsets<F, HASHED, EXACT>(lv[p / P], pt[0], pt[1], pt[2], off[p], fr[p]);
+    }
     // One load per corner. (Measured: serving x-neighbour corners with one 16-byte load plus a
     // range-masked second load halves the throughput, so corners stay separate.)
-    uint32_t q[P][8][F / 2];
+    uint32_t q[N][8][F / 2];
 #pragma unroll
-    for (int p = 0; p < P; p++)
+    for (int p = 0; p < N; p++)
 #pragma unroll
         for (int c = 0; c < 8; c++) load_corner<F>(tab, off[p][c], q[p][c]);
 #pragma unroll
-    for (int p = 0; p < P; p++) {
+    for (int p = 0; p < N; p++) {
         // tcnn's corner weights ((1 * w_x) * w_y) * w_z, the x-y products shared by the z pair.
         const float wx[2] = {1.f - fr[p][0], fr[p][0]}, wy[2] = {1.f - fr[p][1], fr[p][1]};
         const float wz[2] = {1.f - fr[p][2], fr[p][2]};
@@ -165,7 +169,7 @@ __device__ __forceinline__ void gather_operands(const NetArgs& a, __amdgpu_buffe
 #pragma unroll
     for (int l = 0; l < (ND >= 0 ? ND : L); l++) {
         uint32_t r[P * H];
-        gather_level<P, F, BF16, false, EXACT>(a.level[l], tab, pts, r);
+        gather_level<P, F, BF16, false, EXACT>(a.level + l, tab, pts, r);
 #pragma unroll
         for (int p = 0; p < P; p++)
 #pragma unroll
@@ -175,7 +179,7 @@ __device__ __forceinline__ void gather_operands(const NetArgs& a, __amdgpu_buffe
         if constexpr (G == Gather::PHASES) {
             level_phases<L - ND>([&](uint32_t l) {
                 uint32_t r[P * H];
-                gather_level<P, F, BF16, true, false>(a.level[ND + l], tab, pts, r);
+                gather_level<P, F, BF16, true, false>(a.level + ND + l, tab, pts, r);
 #pragma unroll
                 for (int i = 0; i < L - ND; i++)
 #pragma unroll
@@ -187,14 +191,17 @@ __device__ __forceinline__ void gather_operands(const NetArgs& a, __amdgpu_buffe
                         }
             });
         } else {
+            constexpr int NL = G == Gather::PAIRS && (L - ND) % 2 == 0 ? 2 : 1;
 #pragma unroll
-            for (int l = ND; l < L; l++) {
-                uint32_t r[P * H];
-                gather_level<P, F, BF16, true, false>(a.level[l], tab, pts, r);
+            for (int l0 = ND; l0 < L; l0 += NL) {
+                uint32_t r[NL * P * H];
+                gather_level<P, F, BF16, true, false, NL>(a.level + l0, tab, pts, r);
 #pragma unroll
-                for (int p = 0; p < P; p++)
+                for (int l = 0; l < NL; l++)
 #pragma unroll
-                    for (int j = 0; j < H; j++) x[(p * L + l) * H + j] = r[p * H + j];
+                    for (int p = 0; p < P; p++)
+#pragma unroll
+                        for (int j = 0; j < H; j++) x[(p * L + l0 + l) * H + j] = r[(l * P + p) * H + j];
             }
         }
     }
@@ -216,9 +223,9 @@ __device__ __forceinline__ void gather_wide(const NetArgs& a, __amdgpu_buffer_rs
         for (int c = 0; c < 3 * P; c++) pt[c] = __shfl(pts[c], (int)(r + lane % S));
         uint32_t f[P * H];
         if (__all(in_unit_cube<3 * P>(pt)))
-            gather_level<P, F, BF16, false, false>(lv, tab, pt, f);
+            gather_level<P, F, BF16, false, false>(&lv, tab, pt, f);
         else
-            gather_level<P, F, BF16, false, true>(lv, tab, pt, f);
+            gather_level<P, F, BF16, false, true>(&lv, tab, pt, f);
         const bool mine = lane - r < (uint32_t)S;
 #pragma unroll
         for (int p = 0; p < P; p++)
@@ -705,9 +712,9 @@ hipError_t launch_query_k(const NetArgs& a, const RayBatch& rb, uint32_t* queue,
         const hipError_t e = zero_u32(queue, dev::kQueueWords, stream);
         if (e != hipSuccess) return e;
     }
-    // Static launches have few waves per CU: level by level in program order the compiler overlaps
-    // one level's loads with the next one's addresses (65,536 rays 259 against 270 us by phases).
-    const auto few = query_kernel<P, L, F, PREC, PARTS, ND, Gather::LEVELS>();
+    // Static launches have few waves per CU and want loads in flight, not a common level: 48,240
+    // rays 264 us before level order, 246 us by pairs; 65,536 rays 270 us by phases, 259 by levels.
+    const auto few = query_kernel<P, L, F, PREC, PARTS, ND, Gather::PAIRS>();
     const auto k = g.wide ? wide : a.n_dense == (uint32_t)ND ? (g.static_slots ? few : dense) : any;
     hipLaunchKernelGGL(k, dim3(g.blocks), dim3(threads), 0, stream, args, rb, queue);
     return hipGetLastError();

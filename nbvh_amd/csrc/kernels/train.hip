@@ -117,7 +117,7 @@ constexpr uint32_t kSmallBatch = 32768;
 
 // Features of sample l on lanes l (even levels) and l + 32 (odd levels), as the B operands of layer
 // 1: x[s] holds feature 2 s on lanes 0..31 and 2 s + 1 on lanes 32..63 (one v_permlane32_swap per
-// two k-steps). The sums are those of grid_features, corner by corner.
+// two k-steps). Every sum runs over corners 0..7 in order.
 template <int P, int L, int F, bool EXACT>
 __device__ __forceinline__ void half_features(const NetArgs& a, const float* __restrict__ tables, const float* pts,
                                               float* x)
