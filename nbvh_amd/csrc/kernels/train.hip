@@ -26,8 +26,11 @@
 //                    L2 regularisation and dense updates for the matrices, sparse updates
 //                    without L2 for the tables (entries no sample touched keep their value).
 // Gradients are sums over the batch of the per-element gradients divided by n * 8, as the
-// reference's loss kernel writes them; the table gradients (LDS atomics) and the loss are summed
-// in an order that is not fixed.
+// reference's loss kernel writes them; the table gradients are summed by atomics in an order that
+// is not fixed, everything else in a fixed one. Training amplifies that order: four steps of 10,007
+// samples on the 8 x 4 grid, repeated from the same state, give the same first step but for the
+// table gradient's last bits, and then matrices that differ by 2e-8 to 6e-4 (by seed; a ReLU or an
+// L1 sign decided the other way), and losses by 1e-7 to 4e-6.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -75,12 +78,10 @@ __host__ __device__ constexpr int wt_offset(int layer)  // matrix 4 first: the o
     return layer == 4 ? 0 : layer == 3 ? kH * kO : kH * kO + (3 - layer) * kH * kH;
 }
 
-// Also starts the step's loss at zero.
 __global__ __launch_bounds__(256) void train_fragments_kernel(const float* __restrict__ mlp, float* __restrict__ wf,
-                                                              float* __restrict__ wb, float* __restrict__ loss)
+                                                              float* __restrict__ wb)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j == 0) *loss = 0.f;
     if (j >= kMlp) return;
     const int layer = j < w_offset(1) ? 0 : j < w_offset(4) ? 1 + (j - w_offset(1)) / (kH * kH) : 4;
     const int out_w = layer == 4 ? kO : kH, in_w = layer == 0 ? kK0 : kH;
@@ -114,6 +115,7 @@ __global__ __launch_bounds__(256) void train_fragments_kernel(const float* __res
 // that they reach every CU.
 constexpr int kWaveSamples = 32;
 constexpr uint32_t kSmallBatch = 32768;
+constexpr uint32_t kMinGroup   = 2 * kWaveSamples;  // samples of the smaller workgroup
 
 // Features of sample l on lanes l (even levels) and l + 32 (odd levels), as the B operands of layer
 // 1: x[s] holds feature 2 s on lanes 0..31 and 2 s + 1 on lanes 32..63 (one v_permlane32_swap per
@@ -256,9 +258,11 @@ __device__ __forceinline__ void element_loss(int j, float y, float target, bool 
 template <int W>
 __global__ __launch_bounds__(64 * W, 2) void train_backward_kernel(TrainArgs t, const float* __restrict__ wb,
                                                                   const float* __restrict__ targets,
-                                                                  float* __restrict__ act, uint32_t n)
+                                                                  float* __restrict__ act,
+                                                                  double* __restrict__ losses, uint32_t n)
 {
     __shared__ float4 w_lds[kMlp / 4];
+    __shared__ double l_lds[W];
     for (uint32_t j = threadIdx.x; j < (uint32_t)kMlp / 4u; j += 64u * W)
         w_lds[j] = reinterpret_cast<const float4*>(wb)[j];
     const uint32_t lane = threadIdx.x & 63u, g = lane >> 5;
@@ -289,11 +293,20 @@ __global__ __launch_bounds__(64 * W, 2) void train_backward_kernel(TrainArgs t, 
 #pragma unroll
         for (int s = 0; s < kO / 2; s++) row(act, S, kD5 + 2 * s + g, i) = b[s];
     }
-    if (g != 0u) lsum = 0.f;
+    // The workgroup's loss in double, waves in order; train_wgrad_reduce adds the workgroups'. One
+    // float atomic per wave instead: twice as many of them as with 64 samples per wave, in any order
+    // (off by 2 ulp at 65,536 samples).
+    double wsum = g == 0u ? (double)lsum : 0.0;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
-    if (lane == 0) atomicAdd(t.loss, lsum);
+    for (int off = 16; off > 0; off >>= 1) wsum += __shfl_xor(wsum, off);
+    if (lane == 0) l_lds[threadIdx.x >> 6] = wsum;
     __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < W; k++) s += l_lds[k];
+        losses[blockIdx.x] = s;
+    }
     const float* w = reinterpret_cast<const float*>(w_lds);
 #pragma unroll
     for (int layer = 3; layer >= 0; layer--) {  // delta of h(layer + 1)
@@ -730,12 +743,24 @@ __global__ __launch_bounds__(256) void train_wgrad_kernel(const float* __restric
 }
 
 // grad[j] = sum of the chunks' partials: eight running sums over chunks c = r mod 8 (eight loads in
-// flight per thread), added in a fixed order, so the result does not depend on the schedule.
+// flight per thread), added in a fixed order, so the result does not depend on the schedule. The
+// workgroup past the matrix entries adds the n_losses losses of the backward pass, in double: lane
+// t those of t, t + 64, ... in order, then the lanes pairwise.
 __global__ __launch_bounds__(64) void train_wgrad_reduce_kernel(const float* __restrict__ part, uint32_t chunks,
-                                                                float* __restrict__ grad)
+                                                                float* __restrict__ grad,
+                                                                const double* __restrict__ losses, uint32_t n_losses,
+                                                                float* __restrict__ loss)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= kMlp) return;
+    if (j >= kMlp) {
+        static_assert(kMlp % 64 == 0, "the last workgroup has no matrix entries");
+        double s = 0.0;
+        for (uint32_t k = threadIdx.x; k < n_losses; k += 64u) s += losses[k];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+        if (threadIdx.x == 0) *loss = (float)s;
+        return;
+    }
     float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     uint32_t c = 0;
     for (; c + 8 <= chunks; c += 8) {
@@ -786,7 +811,9 @@ uint32_t train_act_stride(uint32_t max_batch) { return (max_batch + 63u) & ~63u;
 
 size_t train_act_bytes(uint32_t max_batch)
 {
-    return ((size_t)dev::kRows * train_act_stride(max_batch) + (size_t)dev::kMlp * (2 + dev::kChunks)) * sizeof(float);
+    const size_t stride = train_act_stride(max_batch);
+    return (dev::kRows * stride + (size_t)dev::kMlp * (2 + dev::kChunks)) * sizeof(float) +
+           stride / dev::kMinGroup * sizeof(double);
 }
 
 hipError_t train_zero(float* p, uint64_t n, hipStream_t stream)
@@ -819,6 +846,7 @@ hipError_t train_gradients(const TrainArgs& t, const float* in, const float* tar
     float* const   wf  = act + (size_t)dev::kRows * S;  // rows of a multiple of 64 floats: 16-byte aligned
     float* const   wb  = wf + dev::kMlp;
     float* const   part = wb + dev::kMlp;
+    double* const  losses = reinterpret_cast<double*>(part + (size_t)dev::kMlp * dev::kChunks);
     const dim3 grid_mlp((dev::kMlp + 255) / 256);
     const bool small = n <= dev::kSmallBatch;
     const uint32_t per_wg = (small ? 2u : 8u) * dev::kWaveSamples;
@@ -889,7 +917,7 @@ hipError_t train_gradients(const TrainArgs& t, const float* in, const float* tar
 #define X(P_, L_, F_)                                                                                                \
     if (a.n_points == P_ && a.n_levels == L_ && a.n_features == F_) {                                                \
         shape = true;                                                                                                \
-        hipLaunchKernelGGL(dev::train_fragments_kernel, grid_mlp, dim3(256), 0, stream, t.mlp, wf, wb, t.loss);      \
+        hipLaunchKernelGGL(dev::train_fragments_kernel, grid_mlp, dim3(256), 0, stream, t.mlp, wf, wb);              \
         if (small)                                                                                                   \
             hipLaunchKernelGGL((dev::train_forward_kernel<P_, L_, F_, 2>), grid, block, 0, stream, t,                \
                                (const float*)wf, in, act, n);                                                        \
@@ -898,10 +926,10 @@ hipError_t train_gradients(const TrainArgs& t, const float* in, const float* tar
                                (const float*)wf, in, act, n);                                                        \
         if (small)                                                                                                   \
             hipLaunchKernelGGL(dev::train_backward_kernel<2>, grid, block, 0, stream, t, (const float*)wb, targets,  \
-                               act, n);                                                                              \
+                               act, losses, n);                                                                      \
         else                                                                                                         \
             hipLaunchKernelGGL(dev::train_backward_kernel<8>, grid, block, 0, stream, t, (const float*)wb, targets,  \
-                               act, n);                                                                              \
+                               act, losses, n);                                                                      \
         if (map.first[L_] > 0)                                                                                       \
             hipLaunchKernelGGL((dev::train_scatter_kernel<P_, L_, F_>), dim3(map.first[L_]), dim3(dev::kScatterThreads), \
                                0, stream, t, map, in, (const float*)act, t.grad_tables, n);                          \
@@ -930,8 +958,8 @@ hipError_t train_gradients(const TrainArgs& t, const float* in, const float* tar
     const uint32_t per = ((n + target - 1) / target + 31u) & ~31u, chunks = (n + per - 1) / per;
     hipLaunchKernelGGL(dev::train_wgrad_kernel, dim3(chunks, dev::kLayers), dim3(256), 0, stream, (const float*)act,
                        (uint32_t)S, n, per, part);
-    hipLaunchKernelGGL(dev::train_wgrad_reduce_kernel, dim3((dev::kMlp + 63) / 64), dim3(64), 0, stream,
-                       (const float*)part, chunks, t.grad_mlp);
+    hipLaunchKernelGGL(dev::train_wgrad_reduce_kernel, dim3(dev::kMlp / 64 + 1), dim3(64), 0, stream,
+                       (const float*)part, chunks, t.grad_mlp, (const double*)losses, grid.x, t.loss);
     return hipGetLastError();
 }
 

@@ -117,7 +117,8 @@ struct TrainArgs {
     const float* tables;
     const float* mlp;
     float*       act;          // workspace: activation rows (720 x act_stride floats), then
-                               // weight fragments and per-chunk matrix-gradient partials
+                               // weight fragments, per-chunk matrix-gradient partials and
+                               // per-workgroup losses
     uint32_t     act_stride;   // samples per activation row (max batch rounded up to 64)
     float*       grad_tables;
     float*       grad_mlp;

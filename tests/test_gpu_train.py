@@ -157,6 +157,117 @@ def test_large_table_gradients_match_oracle(nb, orc, ctx, setup, shape):
     scene.close()
 
 
+@pytest.mark.parametrize("n", [16384, 65536])
+def test_loss_is_the_sum_of_its_samples(nb, ctx, setup, n):
+    """A batch of a power of two divides each element's loss exactly, so the loss is the sum of the
+    losses of its samples as batches of their own, scaled: rounded once, to the nearest float.
+    Bar: half an ulp of the double sum (whose own error is below 1e-12). 16,384 samples go in
+    workgroups of two waves, 65,536 (the same samples four times) in workgroups of eight."""
+    m = 16384
+    x, t = setup["x"][:m], setup["t"][:m]
+    tr = nb.Trainer(ctx, setup["scene"], max_batch=n)
+    loss = tr.step(np.tile(x, (n // m, 1)), np.tile(t, (n // m, 1)), gradients_only=True)
+    from nbvh_amd import hip
+    dx, dt = hip.Buffer.from_array(np.ascontiguousarray(x)), hip.Buffer.from_array(np.ascontiguousarray(t))
+    one = [tr.step_device(dx.ptr + 36 * i, dt.ptr + 32 * i, 1, gradients_only=True) for i in range(m)]
+    exact = np.sum(np.array(one, np.float64)) / m
+    assert abs(loss - exact) <= 0.5 * np.spacing(np.float32(exact)) * (1 + 1e-6), (loss, exact)
+    tr.close()
+
+
+def _fma(a, b, c):
+    """fmaf of float32 arrays: the product is exact in double, the sum is rounded to odd there (the
+    last bit set where it is inexact), so that rounding it to float is the only rounding."""
+    p = a.astype(np.float64) * b.astype(np.float64)
+    c = c.astype(np.float64)
+    s = p + c
+    bb = s - p
+    err = (p - (s - bb)) + (c - bb)
+    bits = s.view(np.int64)
+    up = np.where((err > 0) == (s > 0), 1, -1)
+    return np.where((err != 0) & (bits & 1 == 0), bits + up, bits).view(np.float64).astype(np.float32)
+
+
+def _chain(w, x):
+    """out[n, o] = the fmaf chain of w[o, k] * x[n, k] over k ascending, from zero."""
+    out = np.zeros((x.shape[0], w.shape[0]), np.float32)
+    for k in range(x.shape[1]):
+        out = _fma(np.broadcast_to(w[:, k], out.shape), np.broadcast_to(x[:, k:k + 1], out.shape), out)
+    return out
+
+
+@pytest.mark.parametrize("n", [1063, 33792])
+@pytest.mark.parametrize("shape", [(16, 2, 19, 16, 1.5), (8, 4, 18, 8, 2.0)], ids=["16x2", "8x4"])
+def test_passes_round_like_fmaf_chains(nb, orc, ctx, setup, shape, n):
+    """The matrix-core passes keep the bits of plain fmaf chains: activations over the inputs in
+    order, deltas over the outputs in order, matrix gradients over the samples of a chunk in order
+    (chunks of a multiple of 32 samples, at most 256 of at least 256; the partials in eight running
+    sums). The matrix gradients, which every activation and every delta enters, are compared bit
+    for bit. 33,792 samples (1,024 of them repeated: chunks of 256 start at the same four places)
+    take the large workgroups, 1,063 the small ones and a last tile of 7."""
+    n_levels, n_features, log2, base, scale = shape
+    cfg = nb.network_config(n_levels=n_levels, n_features_per_level=n_features, log2_hashmap_size=log2,
+                            base_resolution=base, per_level_scale=scale)
+    v, tri, _, _, _ = bench_scene(nb)
+    scene = nb.Scene(ctx, v, tri)
+    scene.build_nbvh(256)
+    scene.init_network(cfg, seed=4, table_range=1e-2)
+    _, tables, mlp = scene.network()
+    net = orc.Net(cfg, tables, mlp, *scene.bbox())
+    u = min(n, 1024) if n % 1024 == 0 else n  # distinct samples
+    x, t = setup["x"][:u], setup["t"][:u].astype(np.float32)
+    tr = nb.Trainer(ctx, scene, max_batch=n)
+    tr.step(np.tile(x, (n // u, 1)), np.tile(t, (n // u, 1)), gradients_only=True)
+    got = tr.get(nb.TRAIN_GRAD_MLP)
+    tr.close()
+    f32 = np.float32
+    W = [mlp[a:b].reshape(o, i) for a, b, o, i in ((0, 6144, 64, 96), (6144, 10240, 64, 64), (10240, 14336, 64, 64),
+                                                   (14336, 18432, 64, 64), (18432, 18944, 8, 64))]
+    act = [net.grid(x.reshape(-1, 3), mode=orc.FP32).reshape(u, 96)]
+    for w in W[:4]:
+        act.append(np.maximum(_chain(w, act[-1]), f32(0)))
+    y, z = net.network(x, mode=orc.FP32)
+    assert np.array_equal(_chain(W[4], act[4]), z.astype(f32))
+    y = y.astype(f32)
+    inv_n = f32(1) / (f32(n) * f32(8))
+    keep = t[:, 0] >= 0.5
+    p = np.minimum(np.maximum(y[:, 0], f32(1e-5)), f32(1) - f32(1e-5))
+    g = np.zeros_like(y)
+    g[:, 0] = -(t[:, 0] - p) / (p - p * p)
+    g[:, 1] = np.copysign(f32(1), y[:, 1] - t[:, 1])
+    lin = ((y[:, 2:5] * f32(2) - f32(1)) / f32(0.1)) * f32(0.5) + f32(0.5)
+    g[:, 2:5] = np.copysign(f32(1), lin - t[:, 2:5]) * (f32(1) / f32(0.1))
+    g[:, 5:8] = f32(2) * (y[:, 5:8] - t[:, 5:8]) / (y[:, 5:8] * y[:, 5:8] + f32(1e-2))
+    g[~keep, 1:] = 0
+    delta = [None] * 4 + [(g * inv_n) * (y * (f32(1) - y))]
+    for layer in (3, 2, 1, 0):
+        delta[layer] = np.where(act[layer + 1] > 0, _chain(W[layer + 1].T, delta[layer + 1]), f32(0))
+    target = min(256, (n + 255) // 256)
+    per = ((n + target - 1) // target + 31) // 32 * 32
+    chunks = (n + per - 1) // per
+    if u < n:
+        assert per == 256
+    exp = []
+    for layer in range(5):
+        d, a = delta[layer], act[layer]
+        part = []
+        for c in range(min(chunks, u // per + (u % per != 0))):
+            s = np.zeros((d.shape[1], a.shape[1]), f32)
+            for b in range(c * per, min(u, (c + 1) * per)):
+                s = _fma(np.broadcast_to(d[b][:, None], s.shape), np.broadcast_to(a[b][None], s.shape), s)
+            part.append(s)
+        run, c = [np.zeros_like(part[0]) for _ in range(8)], 0
+        while c + 8 <= chunks:
+            for r in range(8):
+                run[r] = run[r] + part[(c + r) % len(part)]
+            c += 8
+        for c in range(c, chunks):
+            run[0] = run[0] + part[c % len(part)]
+        exp.append((((run[0] + run[1]) + (run[2] + run[3])) + ((run[4] + run[5]) + (run[6] + run[7]))).ravel())
+    assert np.array_equal(got, np.concatenate(exp))
+    scene.close()
+
+
 def test_adam_step_matches_oracle(nb, orc, ctx, setup):
     from oracle import train
     x, t = setup["x"][:2048], setup["t"][:2048]
