@@ -44,6 +44,19 @@ inline QueryGrid query_grid(const RayBatch& rb, uint32_t waves, uint32_t residen
     return QueryGrid{resident, 0u, false};
 }
 
+// Waves per workgroup (of `waves`) that take inputs in a network kernel of at most `resident`
+// workgroups: a batch reaches every CU before a workgroup's second wave is filled; the other waves
+// help to stage the weights and end. A CU's rate is set by the lines its gathers have in flight:
+// eight waves on one CU take seven times as long as one.
+// Measured (us; workgroups of 8 waves filled first / this), FP32, 512 / 4,096 / 16,384 / 32,768 /
+// 65,536 inputs: 16 x 2 grid 237/35 240/50 239/59 240/74 243/124, 8 x 4 118/30 120/37 123/41 123/48
+// 124/67; from 131,072 inputs on every wave works.
+inline uint32_t network_waves(uint32_t n, uint32_t waves, uint32_t resident)
+{
+    const uint32_t need = n / 64u + (n % 64u != 0u ? 1u : 0u), each = need / resident + (need % resident != 0u ? 1u : 0u);
+    return each < waves ? each : waves;
+}
+
 // Dense-prefix length the kernels are specialised for (the hash-only gather of levels >= it):
 // 4 covers the 1024x1024 workload's grid (16 levels, base 16, scale 1.5, 2^19) and the chess
 // configuration (8 levels, base 8, scale 2, 2^18). Other grids take the general gather (ND = -1).

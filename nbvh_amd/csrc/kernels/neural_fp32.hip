@@ -59,18 +59,21 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void neural_query_fp32_kernel(Ne
 }
 
 // tcnn::Network::inference replacement, FP32: in[n x 3P] -> out[n x 8] (sigmoid), logits.
-// Persistent over chunks of blockDim.x inputs (the chunk start is block-uniform, so every wave
-// takes part in each MFMA); the weights are staged once per workgroup.
+// Persistent over chunks of `group` inputs, a multiple of 64 up to blockDim.x (network_waves), so
+// that every lane of a working wave takes part in each MFMA; the weights are staged once per
+// workgroup, by all its waves.
 template <int P, int L, int F, int ND>
 __global__ __launch_bounds__(64 * kF32Waves, 2) void network_fp32_kernel(NetArgs a, const float* __restrict__ in,
-                                                                        uint32_t n, float* __restrict__ out,
+                                                                        uint32_t n, uint32_t group,
+                                                                        float* __restrict__ out,
                                                                         float* __restrict__ logits)
 {
     constexpr int K0 = P * L * F;
     __shared__ float4 w_lds[F32Layout<K0>::FLOATS / 4];
     stage_weights_f32<K0>(a.mlp_f32, w_lds);
     __syncthreads();
-    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
+    if (threadIdx.x >= group) return;
+    for (uint32_t base = blockIdx.x * group; base < n; base += gridDim.x * group) {
         asm volatile("" ::: "memory");  // keeps the weights' LDS reads in the loop (hoisted, they spill)
         const uint32_t i = base + threadIdx.x;
         float x[K0];
@@ -140,9 +143,10 @@ static hipError_t launch_fp32_network_k(const NetArgs& a, const float* in, uint3
     auto k = dev::network_fp32_kernel<P, L, F, ND>;
     constexpr uint32_t threads = 64 * dev::kF32Waves;
     static const uint32_t bpc = blocks_per_cu(k, threads);
-    uint32_t blocks = (n + threads - 1) / threads;
-    blocks = blocks < n_cus * bpc ? blocks : n_cus * bpc;
-    hipLaunchKernelGGL(k, dim3(blocks), dim3(threads), 0, stream, a, in, n, out, logits);
+    const uint32_t resident = n_cus * bpc, group = 64u * network_waves(n, dev::kF32Waves, resident);
+    uint32_t blocks = n / group + (n % group != 0u ? 1u : 0u);
+    blocks = blocks < resident ? blocks : resident;
+    hipLaunchKernelGGL(k, dim3(blocks), dim3(threads), 0, stream, a, in, n, group, out, logits);
     return hipGetLastError();
 }
 
