@@ -51,6 +51,8 @@ inline QueryGrid query_grid(const RayBatch& rb, uint32_t waves, uint32_t residen
 // Measured (us; workgroups of 8 waves filled first / this), FP32, 512 / 4,096 / 16,384 / 32,768 /
 // 65,536 inputs: 16 x 2 grid 237/35 240/50 239/59 240/74 243/124, 8 x 4 118/30 120/37 123/41 123/48
 // 124/67; from 131,072 inputs on every wave works.
+// FP16, 4 waves, 512 / 4,096 / 16,384 / 65,536: 16 x 2 96/16 97/29 94/34 87/86, 8 x 4 22/12 42/17 45/20
+// 44/42.
 inline uint32_t network_waves(uint32_t n, uint32_t waves, uint32_t resident)
 {
     const uint32_t need = n / 64u + (n % 64u != 0u ? 1u : 0u), each = need / resident + (need % resident != 0u ? 1u : 0u);

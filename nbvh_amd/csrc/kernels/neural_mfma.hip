@@ -597,15 +597,18 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void n
 
 template <int P, int L, int F, bool BF16, int ND>
 __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void network_mfma_kernel(NetArgs a, const float* __restrict__ in,
-                                                                           uint32_t n, float* __restrict__ out,
+                                                                           uint32_t n, uint32_t group,
+                                                                           float* __restrict__ out,
                                                                            float* __restrict__ logits)
 {
     constexpr int NF = MlpShape<P * L * F>::N_FRAG;
     __shared__ uint4 wfrag[NF * 64];
     stage_weights<P, L, F, BF16>(a, wfrag);
-    // Persistent over chunks of blockDim.x inputs (the chunk start is block-uniform, so every wave
-    // takes part in each MFMA); the weights are staged once per resident workgroup.
-    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
+    // Persistent over chunks of `group` inputs, a multiple of 64 up to blockDim.x (network_waves), so
+    // that every lane of a working wave takes part in each MFMA; the weights are staged once per
+    // resident workgroup, by all its waves.
+    if (threadIdx.x >= group) return;
+    for (uint32_t base = blockIdx.x * group; base < n; base += gridDim.x * group) {
         asm volatile("" ::: "memory");  // keeps the weights' LDS reads in the loop (hoisted: one wave per SIMD)
         const uint32_t i = base + threadIdx.x;
         float own[3 * P];
@@ -656,12 +659,14 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void n
 
 template <int P, int L, int F, int ND>
 __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void network_fp8_kernel(NetArgs a, const float* __restrict__ in,
-                                                                          uint32_t n, float* __restrict__ out,
+                                                                          uint32_t n, uint32_t group,
+                                                                          float* __restrict__ out,
                                                                           float* __restrict__ logits)
 {
     __shared__ Fp8Lds<P * L * F> w;
     stage_weights_fp8<P * L * F>(a, w);
-    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
+    if (threadIdx.x >= group) return;
+    for (uint32_t base = blockIdx.x * group; base < n; base += gridDim.x * group) {
         asm volatile("" ::: "memory");  // keeps the weights' LDS reads in the loop (hoisted: one wave per SIMD)
         const uint32_t i = base + threadIdx.x;
         float own[3 * P];
@@ -733,10 +738,10 @@ hipError_t launch_network_nd(const NetArgs& a, const float* in, uint32_t n, floa
 {
     auto k = dev::network_mfma_kernel<P, L, F, BF16, ND>;
     static const uint32_t bpc = blocks_per_cu(k, 64 * dev::kWavesPerBlock);
-    const uint32_t per_block = 64 * dev::kWavesPerBlock;
-    uint32_t blocks = (n + per_block - 1) / per_block;
-    blocks = blocks < n_cus * bpc ? blocks : n_cus * bpc;
-    hipLaunchKernelGGL(k, dim3(blocks), dim3(per_block), 0, stream, a, in, n, out, logits);
+    const uint32_t resident = n_cus * bpc, group = 64u * network_waves(n, dev::kWavesPerBlock, resident);
+    uint32_t blocks = n / group + (n % group != 0u ? 1u : 0u);
+    blocks = blocks < resident ? blocks : resident;
+    hipLaunchKernelGGL(k, dim3(blocks), dim3(64 * dev::kWavesPerBlock), 0, stream, a, in, n, group, out, logits);
     return hipGetLastError();
 }
 
@@ -755,10 +760,10 @@ hipError_t launch_network_fp8_nd(const NetArgs& a, const float* in, uint32_t n, 
 {
     auto k = dev::network_fp8_kernel<P, L, F, ND>;
     static const uint32_t bpc = blocks_per_cu(k, 64 * dev::kWavesPerBlock);
-    const uint32_t per_block = 64 * dev::kWavesPerBlock;
-    uint32_t blocks = (n + per_block - 1) / per_block;
-    blocks = blocks < n_cus * bpc ? blocks : n_cus * bpc;
-    hipLaunchKernelGGL(k, dim3(blocks), dim3(per_block), 0, stream, a, in, n, out, logits);
+    const uint32_t resident = n_cus * bpc, group = 64u * network_waves(n, dev::kWavesPerBlock, resident);
+    uint32_t blocks = n / group + (n % group != 0u ? 1u : 0u);
+    blocks = blocks < resident ? blocks : resident;
+    hipLaunchKernelGGL(k, dim3(blocks), dim3(64 * dev::kWavesPerBlock), 0, stream, a, in, n, group, out, logits);
     return hipGetLastError();
 }
 

@@ -150,6 +150,34 @@ def test_small_batches_equal_the_whole(nb, orc, bench, n, precision):
         assert hits_equal(part, whole[start:start + n])
 
 
+@pytest.fixture(scope="module")
+def chess_shape(nb, ctx, bench):
+    """The 8 x 4 grid on the benchmark object."""
+    scene = nb.Scene(ctx, bench["v"], bench["t"])
+    scene.build_nbvh(256)
+    scene.init_network(nb.network_config(n_levels=8, n_features_per_level=4, log2_hashmap_size=18,
+                                         base_resolution=8, per_level_scale=2.0), seed=4, table_range=1e-4)
+    yield nb.NeuralBVHModule(ctx, scene)
+    scene.close()
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp16", "bf16", "fp8"])
+@pytest.mark.parametrize("grid", ["16x2", "8x4"])
+def test_network_batches_equal_the_whole(nb, bench, chess_shape, grid, precision):
+    """The network kernels spread a batch over all CUs before they fill workgroups: outputs and
+    logits at the edges of a wave, of a workgroup and of one, two, four and eight waves on each of
+    256 CUs are those of the same inputs in a batch that fills every workgroup."""
+    mod = bench["module"] if grid == "16x2" else chess_shape
+    prec = {"fp32": nb.PREC_FP32, "fp16": nb.PREC_FP16, "bf16": nb.PREC_BF16, "fp8": nb.PREC_FP8}[precision]
+    x = np.random.default_rng(9).uniform(-0.02, 1.02, (140001, 9)).astype(np.float32)
+    out, logits = mod.network_inference(x, precision=prec)
+    for k in (64, 256, 512, 16384, 32768, 65536, 131072):
+        for n in (k - 1, k, k + 1):
+            o, z = mod.network_inference(x[-n:], precision=prec)
+            assert np.array_equal(o.view(np.uint32), out[-n:].view(np.uint32)), n
+            assert np.array_equal(z.view(np.uint32), logits[-n:].view(np.uint32)), n
+
+
 @pytest.mark.parametrize("any_hit", [False, True])
 def test_neural_query_fp32_bit_exact(nb, orc, bench, any_hit):
     _, rays = camera_rays(nb, orc, 128, 128)
