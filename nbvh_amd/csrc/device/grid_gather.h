@@ -74,5 +74,12 @@ __device__ __forceinline__ void level_phases(const Fn& f)
 template <int L, int ND>
 constexpr Gather kQueryGather = ND >= 0 && L - ND >= 8 ? Gather::PHASES : Gather::LEVELS;
 
+// The network kernels' waves keep step by themselves, so many hashed levels go one at a time; with
+// few of them two at a time.
+// Measured (1M scattered segments, us, levels / pairs): 8 x 4 grid FP16 704 / 683, FP8 731 / 679
+// (all four levels of one point together: 695 / 713); 16 x 2 grid FP16 1678 / 1750, FP8 1735 / 1812.
+template <int L, int ND>
+constexpr Gather kNetworkGather = ND >= 0 && L - ND < 8 ? Gather::PAIRS : Gather::LEVELS;
+
 }  // namespace dev
 }  // namespace nbvh

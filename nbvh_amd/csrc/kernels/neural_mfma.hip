@@ -615,7 +615,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void n
 #pragma unroll
         for (int c = 0; c < 3 * P; c++) own[c] = i < n ? in[(size_t)i * (3 * P) + c] : 0.5f;
         float z[8];
-        mfma_network<P, L, F, BF16, ND, Gather::LEVELS>(a, wfrag, 64u, own, z);
+        mfma_network<P, L, F, BF16, ND, kNetworkGather<L, ND>>(a, wfrag, 64u, own, z);
         if (i < n) {
 #pragma unroll
             for (int j = 0; j < 8; j++) {
@@ -673,7 +673,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void n
 #pragma unroll
         for (int c = 0; c < 3 * P; c++) own[c] = i < n ? in[(size_t)i * (3 * P) + c] : 0.5f;
         float z[8];
-        mfma_network_fp8<P, L, F, ND, Gather::LEVELS>(a, w, 64u, own, z);
+        mfma_network_fp8<P, L, F, ND, kNetworkGather<L, ND>>(a, w, 64u, own, z);
         if (i < n) {
 #pragma unroll
             for (int j = 0; j < 8; j++) {
