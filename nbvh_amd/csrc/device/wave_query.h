@@ -237,6 +237,16 @@ struct RayQueue {
     }
 };
 
+// Position of this workgroup when each XCD has a contiguous range of them: consecutive workgroups
+// are dispatched to the XCDs in turn, and the first gridDim.x % kXcds of these hold one more. A
+// bijection on [0, gridDim.x).
+constexpr uint32_t kXcds = 8;
+__device__ __forceinline__ uint32_t block_by_xcd()
+{
+    const uint32_t x = blockIdx.x % kXcds, odd = gridDim.x % kXcds;
+    return x * (gridDim.x / kXcds) + (x < odd ? x : odd) + blockIdx.x / kXcds;
+}
+
 // First rays of a wave. Static launches (a.static_slots > 0: every ray has a slot) hand ray
 // wave * slots + lane to each lane and never touch the queue; the others start with empty slots
 // and claim. A queued batch whose count (which may live on the device) would give every wave 8
@@ -249,10 +259,13 @@ __device__ __forceinline__ uint32_t first_rays(const NetArgs& a, const RayBatch&
     const uint32_t lane = threadIdx.x & 63u, per_block = blockDim.x >> 6, waves = gridDim.x * per_block;
     if (a.static_slots != 0u) {
         // A count on the device may fill only part of the launch: its rays go to the first wave of
-        // every workgroup, then to the second, so that they reach all CUs; a full launch keeps
-        // neighbouring rays in a workgroup.
+        // every workgroup, then to the second, so that they reach all CUs. A full launch keeps
+        // neighbouring rays on an XCD, as the queue's bands do: their lines share its L2. Measured
+        // (us; the queue before static launches / workgroups in array order / by XCD), FP16: 16 x 2
+        // grid 65,536 rays 220 / 214 / 203, 100,000 312 / 311 / 283, 131,072 341 / 328 / 296; with
+        // 2^21 entries 100,000 rays 363 / 381 / 320; 8 x 4 131,072 rays 214 / 166 / 173.
         const uint32_t w = threadIdx.x >> 6;
-        const uint32_t wave = b.live ? w * gridDim.x + blockIdx.x : blockIdx.x * per_block + w;
+        const uint32_t wave = b.live ? w * gridDim.x + blockIdx.x : block_by_xcd() * per_block + w;
         const uint32_t i = wave * a.static_slots + lane;
         s.state = SLOT_DONE;
         if (lane < a.static_slots && i < q.n_rays) {

@@ -163,6 +163,23 @@ def chess_shape(nb, ctx, bench):
 
 @pytest.mark.parametrize("precision", ["fp32", "fp16", "bf16", "fp8"])
 @pytest.mark.parametrize("grid", ["16x2", "8x4"])
+def test_hand_out_switches_equal_the_whole(nb, orc, bench, chess_shape, grid, precision):
+    """One ray less than, exactly and one more than each batch size at which 256 CUs hand out more
+    rays per wave (2,048 resident waves of 4, 8, 16, 32 and 64 rays) or go over to the queue: the
+    records are those of the same rays in a batch that takes the queue."""
+    mod = bench["module"] if grid == "16x2" else chess_shape
+    prec = {"fp32": nb.PREC_FP32, "fp16": nb.PREC_FP16, "bf16": nb.PREC_BF16, "fp8": nb.PREC_FP8}[precision]
+    _, rays = camera_rays(nb, orc, 512, 400)
+    rays = rays[np.random.default_rng(6).permutation(len(rays))]
+    whole = mod.neural_bvh_traversal(rays, precision=prec, array_order=True)
+    assert (nb.hit_kind(whole) == nb.HIT_NEURAL).mean() > 0.1
+    for k in (8192, 16384, 32768, 65536, 131072):
+        for n in (k - 1, k, k + 1):
+            assert hits_equal(mod.neural_bvh_traversal(rays[:n], precision=prec, array_order=True), whole[:n]), n
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp16", "bf16", "fp8"])
+@pytest.mark.parametrize("grid", ["16x2", "8x4"])
 def test_network_batches_equal_the_whole(nb, bench, chess_shape, grid, precision):
     """The network kernels spread a batch over all CUs before they fill workgroups: outputs and
     logits at the edges of a wave, of a workgroup and of one, two, four and eight waves on each of
@@ -604,6 +621,37 @@ def test_launch_shapes_and_autotune_keep_results(nb, orc, bench):
     with pytest.raises(nb.NbvhError):
         mod.set_launch_shape(nb.PREC_FP16, 0, 0, 2)
     mod.set_launch_shape(nb.PREC_FP16, *saved)
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp16"])
+def test_queued_launch_shapes_keep_results(nb, orc, bench, precision):
+    """A batch beyond one ray per lane of every resident wave goes through the ray queue under each
+    of these shapes: 1, 2, 4 and 8 bands, one workgroup per CU and as many as fit, with and without
+    the image order, and as a two-part launch. The records equal those of the same rays in batches
+    small enough to be handed out by wave index, which never touch the queue."""
+    from nbvh_amd import hip
+    mod = bench["module"]
+    prec = {"fp32": nb.PREC_FP32, "fp16": nb.PREC_FP16}[precision]
+    _, rays = camera_rays(nb, orc, 512, 400)
+    rays = np.concatenate([rays, random_rays(1037, 12, inside_frac=0.4)])
+    ref = np.concatenate([mod.neural_bvh_traversal(rays[i:i + 8192], precision=prec)
+                          for i in range(0, len(rays), 8192)])
+    n, cut, rec = len(rays), 150001, ref.dtype.itemsize
+    dr, dh = hip.Buffer.from_array(rays), hip.Buffer(n * rec)
+    parts = [(dr.ptr, cut, dh.ptr, False), (dr.ptr + cut * 32, n - cut, dh.ptr + cut * rec, False)]
+    saved = mod.launch_shape(prec)
+    try:
+        for bands in (1, 2, 4, 8):
+            for bpc in (1, 0):
+                mod.set_launch_shape(prec, bpc, bands, 0)
+                assert hits_equal(mod.neural_bvh_traversal(rays, precision=prec), ref), (bands, bpc)
+                assert hits_equal(mod.neural_bvh_traversal(rays[:512 * 400], precision=prec, image_width=512),
+                                  ref[:512 * 400]), (bands, bpc)
+                mod.query_parts_device(mod.params(precision=prec), parts)
+                hip.synchronize()
+                assert hits_equal(dh.download(nb.HIT_DTYPE), ref), (bands, bpc)
+    finally:
+        mod.set_launch_shape(prec, *saved)
 
 
 def test_segment_labels_match_oracle(nb, orc, bench):
