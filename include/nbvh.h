@@ -406,7 +406,9 @@ int32_t nbvh_scene_get_launch_shape(const nbvh_scene* scene, uint32_t precision,
 /* Autotuner: times the candidate launch shapes (workgroups per CU in {max, 1, 2, 3} x bands in
  * {1, 2, 4, 8}) of `params` on the given device rays, then, for a batch the coherence order
  * applies to (see ray_order), the fastest shape again with the rays sorted (the sort timed
- * too), and keeps the fastest for the scene and params->precision. Synchronous on `stream`;
+ * too), and keeps the fastest for the scene and params->precision. Shapes that launch this batch
+ * alike are timed once: a batch of at most 64 rays for each resident wave does not use the queue,
+ * and the scene's queue_bands are kept. Synchronous on `stream`;
  * d_hits receives the last run's (shape-independent) hits. best / best_ms may be NULL. */
 int32_t nbvh_autotune(nbvh_ctx* ctx, nbvh_scene* scene, const nbvh_query_params* params, const nbvh_ray* d_rays,
                       uint32_t n_rays, nbvh_hit* d_hits, void* stream, nbvh_launch_shape* best, float* best_ms);

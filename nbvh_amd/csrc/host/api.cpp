@@ -1062,13 +1062,34 @@ NBVH_API int32_t nbvh_scene_get_launch_shape(const nbvh_scene* s, uint32_t preci
 namespace nbvh {
 namespace {
 
+// The grid of a query of n rays with at most bpc workgroups per CU.
+QueryGrid plan_query(const nbvh_ctx* ctx, const nbvh_scene* s, const nbvh_query_params* p, uint32_t n, uint32_t bpc)
+{
+    NetArgs a = neural_args(s, p);
+    a.blocks_per_cu = bpc;
+    const RayBatch batch{nullptr, nullptr, nullptr, 0, n};
+    QueryGrid g{};
+    bool supported = false;
+    if (p->precision == NBVH_PREC_FP32)
+        hip_check(query_fp32(a, batch, nullptr, (uint32_t)ctx->n_cus, nullptr, &supported, &g), "fp32 query plan");
+    else
+        hip_check(query_mfma(a, p->precision, batch, nullptr, (uint32_t)ctx->n_cus, nullptr, &supported, &g),
+                  "mfma query plan");
+    if (!supported) fail(NBVH_ERR_UNSUPPORTED, "no query kernel for this network shape / precision");
+    return g;
+}
+
 // Launch-shape autotuner: persistent workgroups per CU x ray-queue bands, each candidate timed
 // with events over kReps launches of `run` (one query of n rays under the scene's current shape);
 // then the winner in the coherence order where that applies to the batch. The fastest is kept
 // for the scene and precision. The shape only changes which wave traces which ray, never a result.
+// Candidates that launch alike would be told apart by noise alone, and the bands that noise picked
+// would then govern the scene's larger batches: numbers of workgroups that give the same grid are
+// timed once, and where rays are handed out by wave index, which leaves the queue unused, the
+// scene's bands are kept.
 template <typename Run>
-void autotune_batch(nbvh_scene* s, const nbvh_query_params* p, uint32_t n, hipStream_t st, const Run& run,
-                    nbvh_launch_shape* best, float* best_ms)
+void autotune_batch(nbvh_ctx* ctx, nbvh_scene* s, const nbvh_query_params* p, uint32_t n, hipStream_t st,
+                    const Run& run, nbvh_launch_shape* best, float* best_ms)
 {
     hipEvent_t e0, e1;
     hip_check(hipEventCreate(&e0), "hipEventCreate");
@@ -1095,8 +1116,20 @@ void autotune_batch(nbvh_scene* s, const nbvh_query_params* p, uint32_t n, hipSt
         // winner in the coherence order where that would apply by default.
         nbvh_query_params arr = *p;
         if ((arr.flags & NBVH_QUERY_SORT_RAYS) == 0u) arr.flags |= NBVH_QUERY_ARRAY_ORDER;
-        for (uint32_t bpc : {0u, 1u, 2u, 3u})
-            for (uint32_t bands : {1u, 2u, 4u, 8u}) {
+        const bool neural = p->kind == NBVH_QUERY_NEURAL_CLOSEST || p->kind == NBVH_QUERY_NEURAL_ANY;
+        std::vector<QueryGrid> timed;
+        for (uint32_t bpc : {0u, 1u, 2u, 3u}) {
+            std::vector<uint32_t> all_bands = {1u, 2u, 4u, 8u};
+            if (neural) {
+                const QueryGrid g = plan_query(ctx, s, p, n, bpc);
+                if (std::any_of(timed.begin(), timed.end(), [&](const QueryGrid& t) {
+                        return t.blocks == g.blocks && t.static_slots == g.static_slots && t.wide == g.wide;
+                    }))
+                    continue;
+                timed.push_back(g);
+                if (g.static_slots != 0u) all_bands = {saved.queue_bands};
+            }
+            for (uint32_t bands : all_bands) {
                 s->shape[p->precision] = nbvh_launch_shape{bpc, bands, 0u, 0u};
                 const float ms = time_shape(&arr);
                 if (ms < win_ms) {
@@ -1104,6 +1137,7 @@ void autotune_batch(nbvh_scene* s, const nbvh_query_params* p, uint32_t n, hipSt
                     win    = s->shape[p->precision];
                 }
             }
+        }
         if (auto_sort_applies(p, n)) {
             nbvh_query_params srt = *p;
             srt.flags |= NBVH_QUERY_SORT_RAYS;
@@ -1141,7 +1175,7 @@ NBVH_API int32_t nbvh_autotune(nbvh_ctx* ctx, nbvh_scene* s, const nbvh_query_pa
         hip_check(hipSetDevice(ctx->device), "hipSetDevice");
         hipStream_t st = (hipStream_t)stream;
         const RayBatch batch{d_rays, d_hits, nullptr, 0, n};
-        autotune_batch(s, p, n, st, [&](const nbvh_query_params* q) { run_query(ctx, s, q, batch, st); }, best,
+        autotune_batch(ctx, s, p, n, st, [&](const nbvh_query_params* q) { run_query(ctx, s, q, batch, st); }, best,
                        best_ms);
     });
 }
@@ -1160,7 +1194,7 @@ NBVH_API int32_t nbvh_autotune_parts(nbvh_ctx* ctx, nbvh_scene* s, const nbvh_qu
         require(total > 0 && total < (1ull << 32), "the parts hold no rays or more than 2^32 - 1");
         hip_check(hipSetDevice(ctx->device), "hipSetDevice");
         hipStream_t st = (hipStream_t)stream;
-        autotune_batch(s, p, (uint32_t)total, st,
+        autotune_batch(ctx, s, p, (uint32_t)total, st,
                        [&](const nbvh_query_params* q) { run_parts(ctx, s, q, parts, n_parts, st); }, best, best_ms);
     });
 }

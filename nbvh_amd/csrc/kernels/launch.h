@@ -136,15 +136,16 @@ hipError_t path_shade(const PathArgs& a, uint32_t depth, uint32_t n, const uint3
 hipError_t query_triangles(const TriArgs& a, const RayBatch& rb, hipStream_t stream);
 
 // Neural queries (persistent grid sized from n_cus and the kernel's occupancy).
-// *supported = false when no kernel instance matches the network shape.
+// *supported = false when no kernel instance matches the network shape. plan: if not NULL, nothing
+// is launched and the grid that rb would take is written there.
 hipError_t query_fp32(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus, hipStream_t stream,
-                      bool* supported);
+                      bool* supported, QueryGrid* plan = nullptr);
 hipError_t network_fp32(const NetArgs& a, const float* in, uint32_t n, float* out, float* logits, uint32_t n_cus,
                         hipStream_t stream, bool* supported);
 
 // MFMA paths: precision = NBVH_PREC_FP16 / BF16 / FP8.
 hipError_t query_mfma(const NetArgs& a, uint32_t precision, const RayBatch& rb, uint32_t* queue, uint32_t n_cus,
-                      hipStream_t stream, bool* supported);
+                      hipStream_t stream, bool* supported, QueryGrid* plan = nullptr);
 // The network kernels are persistent too: at most n_cus x (resident workgroups per CU) blocks,
 // each staging the weights once.
 hipError_t network_mfma(const NetArgs& a, uint32_t precision, const float* in, uint32_t n, float* out, float* logits,

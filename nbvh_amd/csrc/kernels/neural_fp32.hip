@@ -102,7 +102,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void network_fp32_kernel(NetArgs
 
 template <int P, int L, int F, bool PARTS>
 static hipError_t launch_fp32_query_k(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus,
-                                      hipStream_t stream)
+                                      hipStream_t stream, QueryGrid* plan)
 {
     using dev::Gather;
     constexpr uint32_t threads = 64 * dev::kF32Waves;
@@ -110,6 +110,10 @@ static hipError_t launch_fp32_query_k(const NetArgs& a, const RayBatch& rb, uint
     static const uint32_t bpc = blocks_per_cu(k, threads);
     const uint32_t cap = a.blocks_per_cu != 0u && a.blocks_per_cu < bpc ? a.blocks_per_cu : bpc;
     const QueryGrid g = query_grid(rb, dev::kF32Waves, n_cus * cap, 64u / L < 16u ? 64u / L : 16u, 32u);
+    if (plan) {
+        *plan = g;
+        return hipSuccess;
+    }
     NetArgs args = a;
     args.static_slots = g.static_slots;
     if (g.static_slots == 0u) {
@@ -130,10 +134,10 @@ static hipError_t launch_fp32_query_k(const NetArgs& a, const RayBatch& rb, uint
 
 template <int P, int L, int F>
 static hipError_t launch_fp32_query(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus,
-                                    hipStream_t stream)
+                                    hipStream_t stream, QueryGrid* plan)
 {
-    return rb.parts ? launch_fp32_query_k<P, L, F, true>(a, rb, queue, n_cus, stream)
-                    : launch_fp32_query_k<P, L, F, false>(a, rb, queue, n_cus, stream);
+    return rb.parts ? launch_fp32_query_k<P, L, F, true>(a, rb, queue, n_cus, stream, plan)
+                    : launch_fp32_query_k<P, L, F, false>(a, rb, queue, n_cus, stream, plan);
 }
 
 template <int P, int L, int F, int ND>
@@ -164,12 +168,12 @@ static hipError_t launch_fp32_network(const NetArgs& a, const float* in, uint32_
 #define NBVH_FP32_SHAPES(X) X(3, 16, 2) X(3, 8, 4) X(3, 2, 2) X(3, 4, 2)
 
 hipError_t query_fp32(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus, hipStream_t stream,
-                      bool* supported)
+                      bool* supported, QueryGrid* plan)
 {
     *supported = true;
 #define X(P_, L_, F_)                                                                                    \
     if (a.n_points == P_ && a.n_levels == L_ && a.n_features == F_ && a.n_hidden_layers == 4)            \
-        return launch_fp32_query<P_, L_, F_>(a, rb, queue, n_cus, stream);
+        return launch_fp32_query<P_, L_, F_>(a, rb, queue, n_cus, stream, plan);
     NBVH_FP32_SHAPES(X)
 #undef X
     *supported = false;

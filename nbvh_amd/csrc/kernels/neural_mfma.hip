@@ -699,7 +699,8 @@ auto query_kernel()
 }
 
 template <int P, int L, int F, uint32_t PREC, bool PARTS>
-hipError_t launch_query_k(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus, hipStream_t stream)
+hipError_t launch_query_k(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus, hipStream_t stream,
+                          QueryGrid* plan)
 {
     using dev::Gather;
     constexpr uint32_t threads = 64 * dev::kWavesPerBlock;
@@ -711,6 +712,10 @@ hipError_t launch_query_k(const NetArgs& a, const RayBatch& rb, uint32_t* queue,
     static const uint32_t bpc = blocks_per_cu(any, threads);
     const uint32_t cap = a.blocks_per_cu != 0u && a.blocks_per_cu < bpc ? a.blocks_per_cu : bpc;
     const QueryGrid g = query_grid(rb, dev::kWavesPerBlock, n_cus * cap, 64u / L, 16u);
+    if (plan) {
+        *plan = g;
+        return hipSuccess;
+    }
     NetArgs args = a;
     args.static_slots = g.static_slots;
     if (g.static_slots == 0u) {
@@ -726,10 +731,11 @@ hipError_t launch_query_k(const NetArgs& a, const RayBatch& rb, uint32_t* queue,
 }
 
 template <int P, int L, int F, uint32_t PREC>
-hipError_t launch_query(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus, hipStream_t stream)
+hipError_t launch_query(const NetArgs& a, const RayBatch& rb, uint32_t* queue, uint32_t n_cus, hipStream_t stream,
+                        QueryGrid* plan)
 {
-    return rb.parts ? launch_query_k<P, L, F, PREC, true>(a, rb, queue, n_cus, stream)
-                    : launch_query_k<P, L, F, PREC, false>(a, rb, queue, n_cus, stream);
+    return rb.parts ? launch_query_k<P, L, F, PREC, true>(a, rb, queue, n_cus, stream, plan)
+                    : launch_query_k<P, L, F, PREC, false>(a, rb, queue, n_cus, stream, plan);
 }
 
 template <int P, int L, int F, bool BF16, int ND>
@@ -781,18 +787,18 @@ hipError_t launch_network_fp8(const NetArgs& a, const float* in, uint32_t n, flo
 #define NBVH_MFMA_SHAPES(X) X(3, 16, 2) X(3, 8, 4)
 
 hipError_t query_mfma(const NetArgs& a, uint32_t precision, const RayBatch& rb, uint32_t* queue, uint32_t n_cus,
-                      hipStream_t stream, bool* supported)
+                      hipStream_t stream, bool* supported, QueryGrid* plan)
 {
     *supported = true;
     if (a.n_hidden_layers == 4 && a.mlp_frag != nullptr && a.tables_f16_bytes != 0) {
-#define X(P_, L_, F_)                                                                 \
-    if (a.n_points == P_ && a.n_levels == L_ && a.n_features == F_) {                \
-        if (precision == NBVH_PREC_FP16)                                             \
-            return launch_query<P_, L_, F_, NBVH_PREC_FP16>(a, rb, queue, n_cus, stream);  \
-        if (precision == NBVH_PREC_BF16)                                             \
-            return launch_query<P_, L_, F_, NBVH_PREC_BF16>(a, rb, queue, n_cus, stream);  \
-        if (precision == NBVH_PREC_FP8 && a.mlp_frag_fp8 != nullptr)                 \
-            return launch_query<P_, L_, F_, NBVH_PREC_FP8>(a, rb, queue, n_cus, stream);   \
+#define X(P_, L_, F_)                                                                       \
+    if (a.n_points == P_ && a.n_levels == L_ && a.n_features == F_) {                      \
+        if (precision == NBVH_PREC_FP16)                                                   \
+            return launch_query<P_, L_, F_, NBVH_PREC_FP16>(a, rb, queue, n_cus, stream, plan);  \
+        if (precision == NBVH_PREC_BF16)                                                   \
+            return launch_query<P_, L_, F_, NBVH_PREC_BF16>(a, rb, queue, n_cus, stream, plan);  \
+        if (precision == NBVH_PREC_FP8 && a.mlp_frag_fp8 != nullptr)                       \
+            return launch_query<P_, L_, F_, NBVH_PREC_FP8>(a, rb, queue, n_cus, stream, plan);   \
     }
         NBVH_MFMA_SHAPES(X)
 #undef X

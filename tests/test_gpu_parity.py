@@ -654,6 +654,23 @@ def test_queued_launch_shapes_keep_results(nb, orc, bench, precision):
         mod.set_launch_shape(prec, *saved)
 
 
+def test_autotune_keeps_the_bands_that_a_batch_does_not_use(nb, orc, bench):
+    """A batch handed out by wave index launches alike whatever the number of queue bands: the
+    autotuner has nothing to choose there and keeps the scene's bands for the batches that do."""
+    from nbvh_amd import hip
+    mod = bench["module"]
+    _, rays = camera_rays(nb, orc, 64, 64)
+    dr, dh = hip.Buffer.from_array(rays), hip.Buffer(len(rays) * 48)
+    for prec in (nb.PREC_FP16, nb.PREC_FP32):
+        saved = mod.launch_shape(prec)
+        try:
+            mod.set_launch_shape(prec, 0, 3, 0)
+            (_, bands, _), _ = mod.autotune(mod.params(precision=prec), dr.ptr, len(rays), dh.ptr)
+            assert bands == 3 and mod.launch_shape(prec)[1] == 3
+        finally:
+            mod.set_launch_shape(prec, *saved)
+
+
 def test_segment_labels_match_oracle(nb, orc, bench):
     """GPU label kernel vs the restatement on real segments: visibility and depth bit-exact,
     normals within 1e-7."""
