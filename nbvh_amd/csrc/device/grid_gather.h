@@ -74,6 +74,14 @@ __device__ __forceinline__ void level_phases(const Fn& f)
 template <int L, int ND>
 constexpr Gather kQueryGather = ND >= 0 && L - ND >= 8 ? Gather::PHASES : Gather::LEVELS;
 
+// Next chunk of a persistent network kernel after the one at base < n, or n: base + step may pass 2^32
+// for the last 2^32 - n < step inputs, and must not start again at the first ones.
+__device__ __forceinline__ uint32_t next_chunk(uint32_t base, uint32_t group, uint32_t n)
+{
+    const uint32_t step = gridDim.x * group;
+    return n - base > step ? base + step : n;
+}
+
 // The network kernels' waves keep step by themselves, so many hashed levels go one at a time; with
 // few of them two at a time.
 // Measured (1M scattered segments, us, levels / pairs): 8 x 4 grid FP16 704 / 683, FP8 731 / 679

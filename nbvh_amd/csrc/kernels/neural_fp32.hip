@@ -73,7 +73,7 @@ __global__ __launch_bounds__(64 * kF32Waves, 2) void network_fp32_kernel(NetArgs
     stage_weights_f32<K0>(a.mlp_f32, w_lds);
     __syncthreads();
     if (threadIdx.x >= group) return;
-    for (uint32_t base = blockIdx.x * group; base < n; base += gridDim.x * group) {
+    for (uint32_t base = blockIdx.x * group; base < n; base = next_chunk(base, group, n)) {
         asm volatile("" ::: "memory");  // keeps the weights' LDS reads in the loop (hoisted, they spill)
         const uint32_t i = base + threadIdx.x;
         float x[K0];

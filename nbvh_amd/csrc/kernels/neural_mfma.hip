@@ -608,7 +608,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void n
     // that every lane of a working wave takes part in each MFMA; the weights are staged once per
     // resident workgroup, by all its waves.
     if (threadIdx.x >= group) return;
-    for (uint32_t base = blockIdx.x * group; base < n; base += gridDim.x * group) {
+    for (uint32_t base = blockIdx.x * group; base < n; base = next_chunk(base, group, n)) {
         asm volatile("" ::: "memory");  // keeps the weights' LDS reads in the loop (hoisted: one wave per SIMD)
         const uint32_t i = base + threadIdx.x;
         float own[3 * P];
@@ -666,7 +666,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock, NBVH_MFMA_WAVES_PER_EU) void n
     __shared__ Fp8Lds<P * L * F> w;
     stage_weights_fp8<P * L * F>(a, w);
     if (threadIdx.x >= group) return;
-    for (uint32_t base = blockIdx.x * group; base < n; base += gridDim.x * group) {
+    for (uint32_t base = blockIdx.x * group; base < n; base = next_chunk(base, group, n)) {
         asm volatile("" ::: "memory");  // keeps the weights' LDS reads in the loop (hoisted: one wave per SIMD)
         const uint32_t i = base + threadIdx.x;
         float own[3 * P];
