@@ -6,10 +6,21 @@
 namespace nbvh {
 namespace dev {
 
+// Entries (within the level) of the 8 corners of cell g on a hashed level (a power-of-two size): the
+// coherent prime hash alone, two multiplies per cell, then one xor-and per corner.
+__device__ __forceinline__ void hash_corners(const GridLevel& lv, const uint32_t g[3], uint32_t idx[8])
+{
+    const uint32_t hy0 = g[1] * 2654435761u, hy1 = hy0 + 2654435761u;
+    const uint32_t hz0 = g[2] * 805459861u, hz1 = hz0 + 805459861u;
+    const uint32_t yz[4] = {hy0 ^ hz0, hy1 ^ hz0, hy0 ^ hz1, hy1 ^ hz1};
+    const uint32_t mask = lv.size - 1u, x1 = g[0] + 1u;
+#pragma unroll
+    for (int c = 0; c < 8; c++) idx[c] = (((c & 1) ? x1 : g[0]) ^ yz[c >> 1]) & mask;
+}
+
 // Entries (within the level) of the 8 corners of one level at point (x, y, z), and the fractional
-// position. HASHED: the level is hashed (a power-of-two size), so only the coherent prime hash is
-// formed: two multiplies per level, then one xor-and per corner. The hash of any position is in
-// range, so this form is exact for points outside the unit cube too. Otherwise the general form
+// position. HASHED: the level is hashed, so only hash_corners is formed. The hash of any position is
+// in range, so this form is exact for points outside the unit cube too. Otherwise the general form
 // (dense or hashed at run time, grid_corners) with its EXACT modulo switch.
 template <bool HASHED, bool EXACT>
 __device__ __forceinline__ void level_entries(const GridLevel& lv, float x, float y, float z, uint32_t idx[8],
@@ -18,12 +29,7 @@ __device__ __forceinline__ void level_entries(const GridLevel& lv, float x, floa
     uint32_t g[3];
     grid_cell(lv, x, y, z, g, fr);
     if constexpr (HASHED) {
-        const uint32_t hy0 = g[1] * 2654435761u, hy1 = hy0 + 2654435761u;
-        const uint32_t hz0 = g[2] * 805459861u, hz1 = hz0 + 805459861u;
-        const uint32_t yz[4] = {hy0 ^ hz0, hy1 ^ hz0, hy0 ^ hz1, hy1 ^ hz1};
-        const uint32_t mask = lv.size - 1u, x1 = g[0] + 1u;
-#pragma unroll
-        for (int c = 0; c < 8; c++) idx[c] = (((c & 1) ? x1 : g[0]) ^ yz[c >> 1]) & mask;
+        hash_corners(lv, g, idx);
     } else {
         grid_corners<EXACT>(lv, g, idx);
     }

@@ -334,16 +334,6 @@ __global__ __launch_bounds__(64 * W, 2) void train_backward_kernel(TrainArgs t, 
     }
 }
 
-// Corner entries of a hashed level: grid_corners' coherent-prime hash alone.
-__device__ __forceinline__ void hash_corners(const GridLevel& L, const uint32_t g[3], uint32_t idx[8])
-{
-    const uint32_t hy0 = g[1] * 2654435761u, hy1 = (g[1] + 1u) * 2654435761u;
-    const uint32_t hz0 = g[2] * 805459861u, hz1 = (g[2] + 1u) * 805459861u;
-#pragma unroll
-    for (uint32_t c = 0; c < 8; c++)
-        idx[c] = ((g[0] + (c & 1u)) ^ ((c & 2u) ? hy1 : hy0) ^ ((c & 4u) ? hz1 : hz0)) & (L.size - 1u);
-}
-
 // Work items of the table gradient. Slice j of level l holds the level's entries
 // [j * E, min((j + 1) * E, size)), E = kSliceFloats / F; each slice is split into parts[l] parts
 // of the batch's (sample, point) pairs; level l's items are [first[l], first[l + 1]), item
