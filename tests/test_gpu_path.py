@@ -180,6 +180,28 @@ def test_path_trace_graph_replays_match_eager(nb, setup, hybrid):
         s.destroy()
 
 
+@pytest.mark.parametrize("distance", [6.0, 14.0])
+@pytest.mark.parametrize("precision", ["fp16", "fp32"])
+def test_few_live_paths_of_a_large_frame(nb, setup, precision, distance):
+    """A frame of more pixels than the launch has lanes, so that its bounces' queries take the ray
+    queue with a count on the device, and so few live paths that they are spread over all waves
+    (8 rays per wave and fewer): the image equals that of the bounces with counts on the host."""
+    from nbvh_amd import hip
+    w, h = 512, 320
+    cam = nb.camera_look_at((0, 0, distance), (0, 0, 0), (0, 1, 0), 45.0, w, h)
+    mod = setup["mod"]
+    kw = dict(precision={"fp16": nb.PREC_FP16, "fp32": nb.PREC_FP32}[precision], max_depth=4, rr_start_depth=3)
+    images, counts = [], []
+    for waves in (False, True):
+        acc = hip.Buffer(w * h * 16)
+        counts.append(mod.path_trace_params_device(mod.path_params(w, h, wavefront_bounces=waves, **kw), cam, w, h,
+                                                   acc.ptr))
+        hip.synchronize()
+        images.append(acc.download(np.float32))
+    assert counts[0] == counts[1] and counts[0][0] == w * h and 0 < counts[0][2] <= counts[0][1] <= 8 * 2048
+    assert np.array_equal(images[0], images[1])
+
+
 def test_path_trace_workspace_errors(nb, setup):
     from nbvh_amd import hip
     cam = nb.camera_look_at((0, 0, 3), (0, 0, 0), (0, 1, 0), 45.0, W, H)
