@@ -27,9 +27,14 @@ inline uint32_t blocks_per_cu(K kernel, uint32_t threads)
 // to reset before the launch, no claims, no search for work to steal at the end. rb.n is what
 // counts: with a count on the device (at most n) the waves past it end at once. Larger batches
 // take the queue, on all resident workgroups.
-// Measured (16 x 2 grid, us a call; queue of full waves / WIDE): FP16 4,096 rays 234 / 85, 16,384
-// 243 / 133, 32,384 248 / 196, 65,536 256 / 340 (32 rays per wave: full waves instead); FP32, whose
-// matrix products halve with the second segment block: 65,536 rays 618 / 471.
+// Measured (us a call, camera rays; the queue alone / this rule, with 4,096 / 16,384 / 32,768 /
+// 32,769 / 65,536 / 65,537 / 131,072 / 131,073 rays, either side of each of its lines):
+//   16 x 2 FP16  181/71  181/93  209/146 209/201 220/203 238/257 341/296 342/342
+//   16 x 2 FP32  499/147 598/183 722/239 721/329 772/332 776/503 869/505 868/505
+//   8 x 4 FP16   117/70  118/76  141/110 141/126 170/135 163/135 215/174 216/222
+//   8 x 4 FP32   447/143 445/159 601/213 602/246 674/289 656/370 799/371 801/373
+// FP16 with 32 rays per wave lost (65,536 rays 340 where full waves take 256); FP32's matrix products
+// halve with the second segment block, so it keeps WIDE up to there.
 struct QueryGrid {
     uint32_t blocks, static_slots;
     bool     wide;

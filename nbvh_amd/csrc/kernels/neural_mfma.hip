@@ -89,9 +89,8 @@ __device__ __forceinline__ void load_corner(__amdgpu_buffer_rsrc_t tab, uint32_t
 // Features of all P points of this lane's segment, converted to 16 bits as each level completes:
 // feature k = p*L*F + l*F + f goes to lo[k/8][k%8] (k < K0/2) or hi[(k-K0/2)/8][..]. The FP16
 // tables are read through a buffer resource: 32-bit byte offsets (one VGPR per gather), and the
-// hardware range check returns 0 for any offset past the table instead of faulting. Levels are
-// processed in groups of G: all corner offsets of the group, then all its loads, then the
-// corner weights and the FP32 accumulation over corners 0..7 (tcnn's trilinear weights).
+// hardware range check returns 0 for any offset past the table instead of faulting.
+//
 // Byte offsets of the 8 corners of one level at point (x, y, z) in the whole FP16 table, and the
 // fractional position (level_entries: HASHED and EXACT).
 template <int F, bool HASHED, bool EXACT>
@@ -724,6 +723,8 @@ hipError_t launch_query_k(const NetArgs& a, const RayBatch& rb, uint32_t* queue,
     }
     // Static launches have few waves per CU and want loads in flight, not a common level: 48,240
     // rays 264 us before level order, 246 us by pairs; 65,536 rays 270 us by phases, 259 by levels.
+    // 8 x 4 grid by pairs: 65,536 rays 168 -> 137 us, 131,072 214 -> 166. General grids by pairs: 374
+    // against 381 us (16 x 2 with 2^21 entries, 100,000 rays), others up to 3 % slower; left as they were.
     const auto few = query_kernel<P, L, F, PREC, PARTS, ND, Gather::PAIRS>();
     const auto k = g.wide ? wide : a.n_dense == (uint32_t)ND ? (g.static_slots ? few : dense) : any;
     hipLaunchKernelGGL(k, dim3(g.blocks), dim3(threads), 0, stream, args, rb, queue);

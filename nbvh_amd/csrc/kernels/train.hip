@@ -30,7 +30,7 @@
 // is not fixed, everything else in a fixed one. Training amplifies that order: four steps of 10,007
 // samples on the 8 x 4 grid, repeated from the same state, give the same first step but for the
 // table gradient's last bits, and then matrices that differ by 2e-8 to 6e-4 (by seed; a ReLU or an
-// L1 sign decided the other way), and losses by 1e-7 to 4e-6.
+// L1 sign decided the other way), and losses by up to 4e-6.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -169,7 +169,7 @@ __device__ __forceinline__ void train_layer(const float* w, const float* b, floa
 // device/mlp_f32.h). Per layer the 64 activations of a sample sit in two lanes, k = 2 s + l / 32 in
 // register s, which are stored to the activation rows (128 B per half wave) and feed the next layer.
 // Measured per 65,536 samples of the 16 x 2 grid: 167 us, against 258 us with one thread per
-// sample and weights through the scalar cache; what is left is the gathers and 92 MB of rows.
+// sample and weights through the scalar cache; what is left is the gathers and 94 MB of rows.
 template <int P, int L, int F, int W>
 __global__ __launch_bounds__(64 * W, 2) void train_forward_kernel(TrainArgs t, const float* __restrict__ wf,
                                                                  const float* __restrict__ in,
@@ -254,7 +254,7 @@ __device__ __forceinline__ void element_loss(int j, float y, float target, bool 
 
 // The backward pass, 32 samples per wave like the forward pass: delta of layer l - 1 = W_l^T delta_l
 // where the activation is positive, with the outputs o ascending (the transposed fragments).
-// Measured per 65,536 samples: 102 us (154 us with one thread per sample); 260 MB of rows.
+// Measured per 65,536 samples: 82 us (154 us with one thread per sample); 164 MB of rows.
 template <int W>
 __global__ __launch_bounds__(64 * W, 2) void train_backward_kernel(TrainArgs t, const float* __restrict__ wb,
                                                                   const float* __restrict__ targets,
@@ -294,8 +294,7 @@ __global__ __launch_bounds__(64 * W, 2) void train_backward_kernel(TrainArgs t, 
         for (int s = 0; s < kO / 2; s++) row(act, S, kD5 + 2 * s + g, i) = b[s];
     }
     // The workgroup's loss in double, waves in order; train_wgrad_reduce adds the workgroups'. One
-    // float atomic per wave instead: twice as many of them as with 64 samples per wave, in any order
-    // (off by 2 ulp at 65,536 samples).
+    // float atomic per wave instead: 102 us, and off by 2 ulp at 65,536 samples.
     double wsum = g == 0u ? (double)lsum : 0.0;
 #pragma unroll
     for (int off = 16; off > 0; off >>= 1) wsum += __shfl_xor(wsum, off);
@@ -849,7 +848,8 @@ hipError_t train_gradients(const TrainArgs& t, const float* in, const float* tar
     // >= 16 / 64 / 128 slices and slice scans only (2048 pairs per binning workgroup): 2^19 1.14 /
     // 1.06 / 1.06 / 1.06 ms, 2^20 1.37 / 1.40 / 1.32 / 1.32, 2^21 1.66 / 1.69 / 1.69 / 1.89, 2^22
     // 2.06 / 2.09 / 2.09 / 2.74, 2^23 2.60 / 2.62 / 2.62 / 4.03 (global atomics on the gradient,
-    // the earlier form for the largest tables: 2^22 2.82, 2^23 3.83).
+    // the earlier form for the largest tables: 2^22 2.82, 2^23 3.83), all with one thread per sample
+    // in both passes. On the matrix cores, with 128: 0.81 / 1.09 / 1.37 / 1.73 / 2.27 ms.
 #ifndef NBVH_BIN_MIN_SLICES
 #define NBVH_BIN_MIN_SLICES 128
 #endif
