@@ -598,7 +598,8 @@ def test_scatter_diffuse_matches_oracle(nb, orc, bench, kind):
 
 
 def test_launch_shapes_and_autotune_keep_results(nb, orc, bench):
-    """Every launch shape (workgroups per CU x queue bands x ray order) gives identical hits; the
+    """Every launch shape (workgroups per CU x queue bands x ray order) gives identical hits (a batch
+    of this size is handed out by wave index; the queue's own shapes are tested below); the
     autotuner keeps one of the candidates; a 65,536-ray batch without an image order is sorted
     where the shape says so, and NBVH_QUERY_ARRAY_ORDER keeps array order either way."""
     from nbvh_amd import hip
